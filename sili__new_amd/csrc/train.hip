@@ -15,6 +15,9 @@
 #include "layer.hpp"
 #include "wave.hpp"
 
+#include <cmath>
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace sili {
@@ -117,63 +120,181 @@ __device__ __forceinline__ uint32_t requantize(float w, float imp, bool stochast
     return (wq << 4) | iq;
 }
 
-// Runs t = step(b, x[b], gcol[b]) for b = 0..B-1 in order and adds the sum
-// of t over the wave's lanes into rdx[b].  gcol: one lane's column slice of
-// the feature-major gradient (lanes read different columns).  With
-// B % 4 == 0 the slice is read 8 batch steps at a time as two 16-byte loads,
-// the next group's loads issued before the current group's steps, and the 8
-// steps' t are summed over the lanes together: each lane writes its 8 to
-// sred (512 floats of LDS per wave), each lane then adds one step's values
+// ---- the step without IEEE fix-ups ------------------------------------------
+// A synapse's batch step is bound by VALU issue: of the ~90 instructions that
+// the expressions above compile to, 27 are the IEEE square root and division
+// with their scaling, rounding and special-case selects.  The fast step keeps
+// only what an operand in the middle of the exponent range needs -- the
+// sequences below give the same correctly rounded results there -- and
+// records what the operands' ranges were; a group of steps that met anything
+// else (a tiny, negative, infinite or NaN second moment, a tiny step
+// numerator) is run again from its saved state with the expressions as
+// written.  8192 x 8192, 1.34 M synapses, batch 64: k_train_rows 232 -> 184 us
+// (40 VALU instructions per synapse-step, two of them transcendental);
+// 16384 x 16384, 504 K tiles, batch 256, with the lane layout described at
+// k_train_b4: 6.33 -> 2.80 ms.
+
+// sqrt of x == 0 or x in [2^-80, 2^80]: v_rsq_f32 (1 ulp) and Markstein's
+// correction by the exact remainder x - s*s.  Equal to the IEEE root for every
+// float of [2^-100, 2^101): all 2^23 mantissas at all 201 exponents compared on
+// gfx950.
+__device__ __forceinline__ float mid_sqrt(float x) {
+    const float y = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rsqf(x), 0.0f, 0x1p60f);  // x == 0: s = 0 below
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+// n / d for d in [2^-41, 2^42] and n == 0 or |n| in [2^-80, 2^90]: the
+// reciprocal y refined once, and one correction of the quotient by its exact
+// remainder (Markstein 1990); no exponent scaling.  y is the correctly rounded
+// 1/d (all 2^23 mantissas at 87 exponents compared on gfx950), so n*y is
+// within 1.5 ulp of the quotient and the corrected sum within 1.5 * 2^-24 ulp
+// before its rounding.  Only a quotient that close to the midpoint of two
+// floats could round wrongly; the 11.6 million pairs (n, d) that have one (n *
+// 2^s = M*d/2 +- 1/2, 1 with M odd, enumerated for every d) all gave the IEEE
+// quotient.
+__device__ __forceinline__ float mid_div(float n, float d) {
+    float y = __builtin_amdgcn_rcpf(d);
+    y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+    const float q = n * y;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+// Has v computed at this point (no instruction).  A group's values are used
+// only if no step left the range, and the compiler moves their computation
+// behind that test, keeping every step's operands live up to there (74 spills).
+template <typename T>
+__device__ __forceinline__ void pin_here(T &v) {
+    asm volatile("" : "+v"(v));
+}
+// What a group of fast steps has met: the smallest (bits(v) << 1) - 1 over its
+// second moments and step numerators (zero wraps to the largest value), the
+// largest second moment by its bits (a negative or NaN one compares above
+// every limit).
+struct StepRange {
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+    __device__ __forceinline__ void see(float ema, float n) {
+        const uint32_t e = __builtin_bit_cast(uint32_t, ema);
+        lo = min(min(lo, (e << 1) - 1u), (__builtin_bit_cast(uint32_t, n) << 1) - 1u);
+        hi = max(hi, e);
+    }
+    __device__ __forceinline__ void fold() {
+        pin_here(lo);
+        pin_here(hi);
+    }
+    // every second moment is 0 or in [2^-80, 2^80], every numerator 0 or >= 2^-80
+    __device__ __forceinline__ bool outside() const { return lo < 0x2F000000u || hi > 0x67800000u; }
+};
+// |S| < 2^40: with the second moment's bound on g, the numerator g * S and the
+// quotient stay far from overflow (a NaN or infinite scale fails it).
+__device__ __forceinline__ bool scale_in_range(float S) { return __builtin_fabsf(S) < 0x1p40f; }
+// The parameters for which the fast step is the step: damping on, no decay
+// floor, eps and the cap in the middle of the range.
+inline bool fast_step_params(const TrainParams &p) {
+    const float omb = 1.0f - p.beta2;
+    return p.damp_by_importance != 0 && p.min_decay_frac == 0.0f && p.beta2 >= 0.0f && omb >= 0x1p-20f &&
+           p.eps >= 0x1p-40f && p.eps <= 0x1p10f && p.max_ci >= 0x1p-20f && p.max_ci <= 0x1p40f &&
+           p.max_abs_delta >= 0.0f && std::isfinite(p.max_abs_delta) && std::isfinite(p.lr);
+}
+// One fast step of the importance and the code: the expressions of
+// bounded_update_ci / bounded_update_cw.
+__device__ __forceinline__ void fast_update(float &ci, float &wv, float g, float contrib, float S, float eff_lr,
+                                            float beta2, float omb, float eps, float max_ci, float max_abs_delta,
+                                            StepRange &rg) {
+    const float ema = beta2 * ci + omb * (g * g + contrib * contrib);
+    const float n = -g * S;
+    rg.see(ema, n);
+    ci = __builtin_amdgcn_fmed3f(ema, 0.0f, max_ci);
+    rg.fold();
+    const float raw = mid_div(n, mid_sqrt(ci) + eps);
+    wv = wv + eff_lr * __builtin_amdgcn_fmed3f(raw, -max_abs_delta, max_abs_delta);
+}
+
+// 16-byte load from an address that is 4-byte aligned (a feature-major row of
+// a batch that is no multiple of 4).
+__device__ __forceinline__ float4 load_f4(const float *p) {
+    struct __attribute__((packed, aligned(4))) F4 {
+        float x, y, z, w;
+    };
+    const F4 v = *reinterpret_cast<const F4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// The lanes' 8 terms of batch steps b0..b0+7 (lane l's in sred[8 l ..])
+// summed over the lanes into rdx[b0..b0+n): each lane adds one step's values
 // of 8 lanes (read in a rotated order so that the wave's 64 reads hit 64
 // different banks), and three exchanges combine the 8 groups.
-template <typename Step>
+__device__ __forceinline__ void reduce8(const float *sred, float *rdx, int64_t b0, uint32_t n) {
+    const uint32_t lane = __lane_id(), j = lane & 7u, grp = lane >> 3;
+    wave_lds_sync();
+    float sum = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) sum += sred[(grp * 8u + ((i + grp) & 7u)) * 8u + j];
+    sum += __shfl_xor(sum, 8, 64);
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (lane < n) rdx[b0 + lane] += sum;
+    wave_lds_sync();
+}
+
+// Runs a lane's batch steps b = 0..B-1 in order over its column slice gcol of
+// the feature-major gradient (lanes read different columns) and adds the sum
+// of the lanes' dx terms per step into rdx[b]: 8 steps at a time as two
+// 16-byte loads (the next group's issued before this group's steps), then 4,
+// then one by one.  step(mode, b, x, dy) returns the dx term; mode 0 takes the
+// step as written, the others (the caller's `mode`, uniform over the wave) are
+// fast ones: save() and back() keep and restore the lane's state around a
+// group of them, and redo() says, for the whole wave, that the group must be
+// run as written.  sx: 16-byte aligned.
+template <typename Step, typename Save, typename Back, typename Redo>
 __device__ __forceinline__ void batch_steps(const float *__restrict__ gcol, int64_t B, const float *sx, float *rdx,
-                                            float *sred, Step &step) {
+                                            float *sred, int mode, Step &step, Save &save, Back &back, Redo &redo) {
     const uint32_t lane = __lane_id();
-    if ((B & 3) == 0) {
-        const float4 *g4 = reinterpret_cast<const float4 *>(gcol);
-        const float4 z4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        float4 n0 = g4[0];
-        float4 n1 = B > 4 ? g4[1] : z4;
-        const uint32_t j = lane & 7u, grp = lane >> 3;
-        // lanes' 8 terms of batch steps b0..b0+7 summed into rdx[b0..]
-        auto reduce8 = [&](int64_t b0, const float (&t)[8]) {
-            float4 *w4 = reinterpret_cast<float4 *>(sred + lane * 8);
-            w4[0] = make_float4(t[0], t[1], t[2], t[3]);
-            w4[1] = make_float4(t[4], t[5], t[6], t[7]);
-            wave_lds_sync();
-            float sum = 0.0f;
+    float *mine = sred + lane * 8;
+    auto fast_group = [&](auto steps, auto m, int64_t b0, const float4 &c0, const float4 &c1) -> bool {
+        constexpr int N = decltype(steps)::value;
+        save();
+        const float4 x0 = reinterpret_cast<const float4 *>(sx + b0)[0];
+        const float4 x1 = N == 8 ? reinterpret_cast<const float4 *>(sx + b0)[1] : x0;
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        const float d[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        float t[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) sum += sred[(grp * 8u + ((i + grp) & 7u)) * 8u + j];
-            sum += __shfl_xor(sum, 8, 64);
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
-            if (lane < 8u && b0 + lane < B) rdx[b0 + lane] += sum;
-            wave_lds_sync();
-        };
-        const int64_t full = B & ~(int64_t)7;
-        for (int64_t b0 = 0; b0 < full; b0 += 8) {
-            const float4 c0 = n0, c1 = n1;
-            if (b0 + 8 < B) n0 = g4[(b0 + 8) >> 2];
-            if (b0 + 12 < B) n1 = g4[(b0 + 12) >> 2];
-            const float d[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-            float t[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) t[q] = step(b0 + q, sx[b0 + q], d[q]);
-            reduce8(b0, t);
+        for (int q = 0; q < N; ++q) t[q] = step(m, b0 + q, x[q], d[q]);
+        reinterpret_cast<float4 *>(mine)[0] = make_float4(t[0], t[1], t[2], t[3]);
+        reinterpret_cast<float4 *>(mine)[1] = make_float4(t[4], t[5], t[6], t[7]);
+        if (!redo()) return true;
+        back();
+        return false;
+    };
+    auto group = [&](auto steps, int64_t b0, const float4 &c0, const float4 &c1) {
+        constexpr int N = decltype(steps)::value;
+        bool done = false;
+        if (mode == 2) done = fast_group(steps, std::integral_constant<int, 2>{}, b0, c0, c1);
+        else if (mode == 1) done = fast_group(steps, std::integral_constant<int, 1>{}, b0, c0, c1);
+        if (!done) {
+#pragma unroll 1
+            for (int q = 0; q < N; ++q)
+                mine[q] = step(std::integral_constant<int, 0>{}, b0 + q, sx[b0 + q], gcol[b0 + q]);
+            if (N < 8) reinterpret_cast<float4 *>(mine)[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
-        if (B & 4) {  // last 4 steps (loaded by the last full group, or up front)
-            const float d[4] = {n0.x, n0.y, n0.z, n0.w};
-            float t[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) t[q] = step(full + q, sx[full + q], d[q]);
-            reduce8(full, t);
-        }
-    } else {
-        for (int64_t b = 0; b < B; ++b) {
-            const float tot = wave_sum(step(b, sx[b], gcol[b]));
-            if (lane == 0u) rdx[b] = rdx[b] + tot;
-        }
+        reduce8(sred, rdx, b0, N);
+    };
+    const float4 z4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 n0 = B >= 4 ? load_f4(gcol) : z4;
+    float4 n1 = B >= 8 ? load_f4(gcol + 4) : z4;
+    int64_t b0 = 0;
+    for (; b0 + 8 <= B; b0 += 8) {
+        const float4 c0 = n0, c1 = n1;
+        if (b0 + 12 <= B) n0 = load_f4(gcol + b0 + 8);
+        if (b0 + 16 <= B) n1 = load_f4(gcol + b0 + 12);
+        group(std::integral_constant<int, 8>{}, b0, c0, c1);
+    }
+    if (b0 + 4 <= B) {
+        group(std::integral_constant<int, 4>{}, b0, n0, z4);
+        b0 += 4;
+    }
+    for (; b0 < B; ++b0) {
+        const float tot = wave_sum(step(std::integral_constant<int, 0>{}, b0, sx[b0], gcol[b0]));
+        if (lane == 0u) rdx[b0] = rdx[b0] + tot;
     }
 }
 
@@ -196,6 +317,7 @@ struct TrainArgs {
     float lr, beta2, eps, min_decay_frac, max_abs_delta, max_ci, zero_escape_eps;
     int lr_per_row_nnz, damp, stochastic;
     int deferred, no_scale;    // DeferredScaleWrite; NoScalePolicy
+    int fast;                  // fast_step_params
     uint64_t seed;             // this call's stochastic-rounding seed
 };
 
@@ -212,7 +334,7 @@ struct TrainArgs {
 //     stepped by g; scale gradients weigh by the stored code, component 0
 //     only; (cw, ci) are kept for k_train_store (linear_disldo.hpp:687-790).
 template <int RANK, bool DEFERRED, bool COLS>
-__global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
+__global__ __launch_bounds__(256, RANK == 1 ? 4 : 2) void k_train_rows(TrainArgs a) {
     __shared__ double s_part[WAVES_T][64][2 * RANK];
     extern __shared__ __attribute__((aligned(16))) float s_dyn[];  // [wave][dx B | x B]
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
@@ -225,9 +347,10 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
         for (int64_t b = lane; b < B; b += 64) a.dx[b * a.n_in + r] = 0.0f;
         return;
     }
-    float *rdx = s_dyn + (int64_t)wave * (2 * B + 512);
-    float *sx = rdx + B;       // the row's inputs, read by every lane
-    float *sred = sx + B;      // dx reduction staging (batch_steps)
+    const int64_t BP = (B + 3) & ~(int64_t)3;  // sred is read and written 16 bytes at a time
+    float *rdx = s_dyn + (int64_t)wave * (2 * BP + 512);
+    float *sx = rdx + BP;      // the row's inputs, read by every lane
+    float *sred = sx + BP;     // dx reduction staging (batch_steps)
     const float *xrow = a.xT + r * B;
     for (int64_t b = lane; b < B; b += 64) {
         rdx[b] = 0.0f;
@@ -277,31 +400,76 @@ __global__ __launch_bounds__(256) void k_train_rows(TrainArgs a) {
             psg[k] = psgc[k] = 0.0;
             pm[k] = pmc[k] = 0.0f;
         }
+        // every output scale of the chunk 1: the fp64 terms' product by it is
+        // exact, and so is code * gradient (48 bits), so the sum is one fma
+        const bool os1 = RANK == 1 && __all(!has || os_k[0] == 1.0f);
+        const bool ok = !has || scale_in_range(S_step);
+        StepRange rg;
         // one batch step of this lane's synapse (b in order); lanes without
         // a synapse step zeros (finite throughout) and contribute nothing
-        auto step = [&](int64_t b, float iv, float dy_raw) -> float {
-            const float dyv = has ? dy_raw : 0.0f;
+        auto step = [&](auto m, int64_t b, float iv, float dy_raw) -> float {
+            // (a fast step of a lane without a synapse may meet anything: its
+            // term is dropped below, its sums and bytes after the steps)
+            const float dyv = decltype(m)::value != 0 || has ? dy_raw : 0.0f;
             const float g = dyv * iv;
-            {
-                const float contrib = iv * cw_orig;
+            const float contrib = iv * cw_orig;
+            if constexpr (decltype(m)::value != 0) {
+                fast_update(ci, wv, g, contrib, S_step, eff_lr, a.beta2, 1.0f - a.beta2, a.eps, a.max_ci,
+                            a.max_abs_delta, rg);
+            } else {
                 ci = bounded_update_ci(ci, g, contrib, a.beta2, a.min_decay_frac, a.max_ci);
                 wv = wv + bounded_update_cw(g, ci, S_step, eff_lr, a.eps, a.damp != 0, a.max_abs_delta);
-                cw = deferred ? wv : wv * S;
-                const float qf = deferred ? cw_orig : ((wv == 0.0f) ? a.zero_escape_eps : wv);
+            }
+            cw = deferred ? wv : wv * S;
+            const float qf = deferred ? cw_orig : ((wv == 0.0f) ? a.zero_escape_eps : wv);
+            if constexpr (decltype(m)::value == 2) {
+                psg[0] = __builtin_fma((double)qf, (double)g, psg[0]);
+                psgc[0] = __builtin_fma((double)qf, (double)contrib, psgc[0]);
+            } else {
 #pragma unroll
                 for (int k = 0; k < nk; ++k) {
                     psg[k] = psg[k] + ((double)qf * (double)os_k[k]) * (double)g;
                     psgc[k] = psgc[k] + ((double)qf * (double)os_k[k]) * (double)contrib;
-                    if constexpr (COLS) {
-                        pm[k] = pm[k] + (qf * vs_k[k]) * g;
-                        pmc[k] = pmc[k] + (qf * vs_k[k]) * contrib;
-                    }
+                }
+            }
+            if constexpr (COLS) {
+#pragma unroll
+                for (int k = 0; k < nk; ++k) {
+                    pm[k] = pm[k] + (qf * vs_k[k]) * g;
+                    pmc[k] = pmc[k] + (qf * vs_k[k]) * contrib;
                 }
             }
             // dx[b][row]: this synapse's term
             return has ? cw * dyv : 0.0f;
         };
-        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, step);
+        float ci_0, wv_0, pm_0[RANK], pmc_0[RANK];
+        double psg_0[RANK], psgc_0[RANK];
+        auto save = [&]() {
+            rg = StepRange{};
+            ci_0 = ci;
+            wv_0 = wv;
+#pragma unroll
+            for (int k = 0; k < RANK; ++k) {
+                psg_0[k] = psg[k];
+                psgc_0[k] = psgc[k];
+                pm_0[k] = pm[k];
+                pmc_0[k] = pmc[k];
+            }
+        };
+        auto back = [&]() {
+            ci = ci_0;
+            wv = wv_0;
+#pragma unroll
+            for (int k = 0; k < RANK; ++k) {
+                psg[k] = psg_0[k];
+                psgc[k] = psgc_0[k];
+                pm[k] = pm_0[k];
+                pmc[k] = pmc_0[k];
+            }
+        };
+        auto redo = [&]() -> bool { return __any(has && rg.outside()); };
+        const int mode = a.fast && __all(ok) ? (os1 ? 2 : 1) : 0;
+        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, mode, step, save, back, redo);
         if (has) {
             if (deferred) {
                 a.def_w[vb] = wv;
@@ -425,9 +593,10 @@ __global__ __launch_bounds__(256) void k_sparse_train_rows(SparseTrainArgs a) {
         if (lane == 0u) a.rowsum[2 * r] = a.rowsum[2 * r + 1] = 0.0;
         return;
     }
-    float *rdx = s_dyn + (int64_t)wave * (2 * B + 512);
-    float *sx = rdx + B;
-    float *sred = sx + B;
+    const int64_t BP = (B + 3) & ~(int64_t)3;
+    float *rdx = s_dyn + (int64_t)wave * (2 * BP + 512);
+    float *sx = rdx + BP;
+    float *sred = sx + BP;
     const float *xrow = a.xT + r * B;
     for (int64_t b = lane; b < B; b += 64) {
         rdx[b] = 0.0f;
@@ -453,7 +622,7 @@ __global__ __launch_bounds__(256) void k_sparse_train_rows(SparseTrainArgs a) {
         const float combined_imp_scale = imp_scale * out_imp_scale;
         double psg = 0.0, psgc = 0.0;
         // lanes whose synapse has no dy entry at b compute and discard
-        auto step = [&](int64_t b, float iv, float dy_raw) -> float {
+        auto step = [&](auto, int64_t b, float iv, float dy_raw) -> float {
             const float dyv = has ? dy_raw : 0.0f;
             const bool present = __builtin_bit_cast(uint32_t, dyv) != 0u;
             const float w_stored = fp4_decode(byte >> 4);
@@ -469,7 +638,9 @@ __global__ __launch_bounds__(256) void k_sparse_train_rows(SparseTrainArgs a) {
             psgc = psgc + (present ? ((double)w_stored * (double)out_scale) * (double)contrib : 0.0);
             return present ? w * dyv : 0.0f;
         };
-        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, step);
+        auto nothing = []() {};
+        auto never = []() -> bool { return false; };
+        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, 1, step, nothing, nothing, never);
         if (has) a.val[vb] = (uint8_t)byte;
         s_part[wave][lane][0] = has ? psg : 0.0;
         s_part[wave][lane][1] = has ? psgc : 0.0;
@@ -519,8 +690,7 @@ __global__ __launch_bounds__(256) void k_sparse_train_vs(const uint32_t *__restr
 
 // ---- block4 tiles ------------------------------------------------------------------
 struct B4TrainArgs {
-    const uint32_t *byte_start, *tile_start;  // canonical block4 store
-    const uint8_t *idx;
+    const uint32_t *tile_start, *tcol;  // canonical block4 store; the tiles' block columns
     uint8_t *tiles;
     int64_t brows, n_in, n_out, B, nnz_scattered;
     const float *xT, *gT;
@@ -531,195 +701,292 @@ struct B4TrainArgs {
     float *b4term;             // [tiles * 16][2 * rank] or NULL
     float lr, beta2, eps, min_decay_frac, max_abs_delta, max_ci, zero_escape_eps;
     int lr_per_row_nnz, damp, stochastic;
+    int fast;                  // fast_step_params
     uint64_t seed;
 };
 
-// One wave per canonical block row (linear_disldo.hpp:962-1951, FP4): every
-// slot of the row's tiles trains.  Lanes hold 4 tiles x 16 slots, ordered
-// (tile, li, lj) so a quad is one tile row.  A tile whose 4 columns are all
-// in range sums its row's 4 row-gradient and dx terms per batch step in lane
-// order ((t0 + t1) + t2) + t3 in fp32 (the reference's 4-lane path); an
-// edge tile adds its fp64 row-gradient terms one by one (its scalar path).
-// The tiles' fp64 row partials are added in tile order; then the block
-// rows' scale step.
-// Lane J of the calling lane's quad (DPP quad_perm, a VALU move).
-template <int J>
-__device__ __forceinline__ float quad_lane(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), J * 0x55, 0xF, 0xF, false));
-}
-template <int J>
-__device__ __forceinline__ double quad_lane(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, J * 0x55, 0xF, 0xF, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), J * 0x55, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-// ((l0 + l1) + l2) + l3 over the quad, on every lane of it
-template <typename T>
-__device__ __forceinline__ T quad_sum(T v) {
-    return ((quad_lane<0>(v) + quad_lane<1>(v)) + quad_lane<2>(v)) + quad_lane<3>(v);
-}
+// One block of 4 waves per canonical block row (linear_disldo.hpp:962-1951,
+// FP4): every slot of the row's tiles trains.  A lane holds one tile row
+// (lane = 4 * tile + li; a wave takes 16 tiles at a time, the block 64): its
+// 4 slots are 4 independent chains of batch steps, and the sums over a tile
+// row that the reference's 4-lane path forms, ((t0 + t1) + t2) + t3 in fp32
+// per batch step for the row gradient, stay inside the lane.  (A slot per lane
+// with the sums by quad moves spent 21 of its 87 instructions per slot-step on
+// them, and each batch step added its dx terms to LDS by itself.)  An edge
+// tile, whose 4 columns are not all in range, adds its fp64 row-gradient terms
+// one by one (the reference's scalar path).  The tiles' fp64 row partials are
+// added in tile order; then the block rows' scale step.  dx: per 4 batch steps
+// the lanes' sums of a DPP row's 4 tiles go to the wave's own LDS rows by one
+// add per lane; the waves' rows are added in wave order at the end.
+constexpr uint32_t WAVES_B4 = 4;  // waves per block of k_train_b4
+constexpr uint32_t TILES_B4 = 16 * WAVES_B4;  // tiles the block takes at a time
+// Floats of a row of batch values in LDS: 16-byte aligned, and 4 more so that
+// the 4 rows' reads of one step group fall into different banks.
+__host__ __device__ inline int64_t b4_ld(int64_t B) { return ((B + 3) & ~(int64_t)3) + 4; }
 
-constexpr uint32_t WAVES_B4 = 2;  // waves per block of k_train_b4 (LDS: 4 rows x B floats per wave)
+// A lane's state while its 4 slots train.
+template <int RANK, bool COLS>
+struct B4State {
+    float q[4], ci[4];
+    double mr[2 * RANK];
+    float mc[COLS ? 4 : 1][2 * RANK];
+};
 
-template <int RANK>
-__global__ __launch_bounds__(128) void k_train_b4(B4TrainArgs a) {
-    __shared__ uint32_t s_bc[WAVES_B4][64];
-    __shared__ double s_mr[WAVES_B4][4][4][2 * RANK];  // [tile][li][k | contrib k]
-    extern __shared__ float s_dxb[];                    // [wave][li][B]: the block row's dx terms
+template <int RANK, bool COLS>
+__global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4TrainArgs a) {
+    __shared__ double s_mr[TILES_B4][4][2 * RANK];  // [tile][li][k | contrib k]
+    __shared__ double s_row[4][2 * RANK];           // the rows' sums over all tiles
+    extern __shared__ __attribute__((aligned(16))) float s_dyn[];  // x [4][LD], then dx [wave][4][LD]
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const int64_t br = (int64_t)blockIdx.x * WAVES_B4 + wave;
-    if (br >= a.brows) return;
+    const int64_t br = blockIdx.x;
     const uint32_t t0 = a.tile_start[br], t1 = a.tile_start[br + 1];
-    if (t0 == t1) return;
-    const int64_t B = a.B;
-    float *sdx = s_dxb + (int64_t)wave * 4 * B;
-    for (int64_t i = lane; i < 4 * B; i += 64) sdx[i] = 0.0f;
-    wave_lds_sync();
+    if (t0 == t1) return;  // the whole block
+    const int64_t B = a.B, LD = b4_ld(B);
+    float *sx = s_dyn, *sdx = s_dyn + (1 + wave) * 4 * LD;
+    for (int64_t i = threadIdx.x; i < 4 * LD; i += 256) {
+        const int64_t l = i / LD, b = i % LD;
+        sx[i] = b < B && br * 4 + l < a.n_in ? a.xT[(br * 4 + l) * B + b] : 0.0f;
+    }
+    for (int64_t i = lane; i < 4 * LD; i += 64) sdx[i] = 0.0f;
+    if (threadIdx.x < 8u * RANK) (&s_row[0][0])[threadIdx.x] = 0.0;
+    __syncthreads();
     const uint32_t nnz_row = (t1 - t0) * 4u;
     const float eff_lr = a.lr_per_row_nnz ? a.lr / (float)nnz_row : a.lr;
-    const uint32_t tl = lane >> 4, li = (lane >> 2) & 3u, lj = lane & 3u;
+    const float omb = 1.0f - a.beta2;
+    const uint32_t tl = lane >> 2, li = lane & 3u;
     const int64_t row = br * 4 + li;
     const bool row_ok = row < a.n_in;
-    double rowacc[2 * RANK];  // lanes 0..3: row br*4 + lane
+    float vs_k[RANK];
 #pragma unroll
-    for (int k = 0; k < 2 * RANK; ++k) rowacc[k] = 0.0;
-    uint32_t pos = a.byte_start[br], carry = 0, ebase = t0;
-    const uint32_t end = a.byte_start[br + 1];
-    while (pos < end) {
-        const Chunk ch = decode_chunk(a.idx, pos, end, carry);
-        if (ch.T == 0ull) break;
-        if (ch.term) s_bc[wave][ch.rank] = ch.col;
-        wave_lds_sync();
-        const uint32_t nt = (uint32_t)__popcll(ch.T);
-        for (uint32_t sub = 0; sub < nt; sub += 4) {
-            const uint32_t trank = sub + tl;
-            const bool tile_ok = trank < nt;
-            const uint32_t bc = tile_ok ? s_bc[wave][trank] : 0u;
-            const int64_t t = (int64_t)ebase + trank;
-            const int64_t col = (int64_t)bc * 4 + lj;
-            const bool has = tile_ok && row_ok && col < a.n_out;
-            const bool full = tile_ok && (int64_t)bc * 4 + 4 <= a.n_out;
-            const uint32_t slot = lj * 4u + li;
-            const uint32_t byte = has ? (uint32_t)a.tiles[t * 16 + slot] : 0u;
-            float vs_k[RANK], os_k[RANK];
-            float S = 0.0f;
+    for (int k = 0; k < RANK; ++k) vs_k[k] = row_ok ? a.vs[row * RANK + k] : 0.0f;
+    const float imp_scale = (a.is && row_ok) ? a.is[row] : 1.0f;
+    const float *xl = sx + li * LD;
+    for (uint32_t p0 = t0; p0 < t1; p0 += TILES_B4) {
+        const uint32_t tw = p0 + wave * 16u;  // the wave's first tile
+        if (tw < t1) {
+            const bool tile_ok = tw + tl < t1;
+            const uint32_t t = tile_ok ? tw + tl : tw;  // a lane past the end steps a copy that it drops
+            const int64_t c0 = (int64_t)a.tcol[t] * 4;
+            const bool full = c0 + 4 <= a.n_out;
+            const uint4 tb = *reinterpret_cast<const uint4 *>(a.tiles + (uint64_t)t * 16);
+            const uint32_t word[4] = {tb.x, tb.y, tb.z, tb.w};
+            B4State<RANK, COLS> s;
+            float q0[4], S[4], os_k[4][RANK];
+            bool has[4], ok = true;
+            const float *g0 = a.gT + c0 * B;  // slot j's gradient row: g0 + j * B (c0 < n_out)
 #pragma unroll
-            for (int k = 0; k < RANK; ++k) {
-                vs_k[k] = row_ok ? a.vs[row * RANK + k] : 0.0f;
-                os_k[k] = has ? a.os[col * RANK + k] : 0.0f;
-                S = S + vs_k[k] * os_k[k];
-            }
-            const float imp_scale = (a.is && row_ok) ? a.is[row] : 1.0f;
-            const float cis = imp_scale * ((a.ois && has) ? a.ois[col] : 1.0f);
-            const float q0 = fp4_decode(byte & 0xFu);
-            float q = q0;
-            float ci = fp4_decode(byte >> 4) * cis;
-            double mr[2 * RANK];
-            float mc[2 * RANK];
-#pragma unroll
-            for (int k = 0; k < 2 * RANK; ++k) {
-                mr[k] = 0.0;
-                mc[k] = 0.0f;
-            }
-            const float *xrow = a.xT + (row_ok ? row : 0) * B;
-            const float *gcol = a.gT + (has ? col : 0) * B;
-            // one batch step of this lane's slot (b in order)
-            auto step = [&](int64_t b, float iv_raw, float dy_raw) {
-                const float iv = row_ok ? iv_raw : 0.0f;
-                const float dyv = has ? dy_raw : 0.0f;
-                const float g = dyv * iv;
-                const float contrib = q0 * iv;
-                ci = bounded_update_ci(ci, g, contrib, a.beta2, a.min_decay_frac, a.max_ci);
-                q = q + bounded_update_cw(g, ci, S, eff_lr, a.eps, a.damp != 0, a.max_abs_delta);
-                const float qf = (q == 0.0f) ? a.zero_escape_eps : q;
-                const float tdx = has ? (q * S) * dyv : 0.0f;
+            for (int j = 0; j < 4; ++j) {
+                has[j] = tile_ok && row_ok && c0 + j < a.n_out;
+                const int64_t col = has[j] ? c0 + j : 0;
+                const uint32_t byte = has[j] ? (word[j] >> (8u * li)) & 0xFFu : 0u;
+                S[j] = 0.0f;
 #pragma unroll
                 for (int k = 0; k < RANK; ++k) {
-                    mc[k] = mc[k] + (qf * vs_k[k]) * g;
-                    mc[RANK + k] = mc[RANK + k] + (qf * vs_k[k]) * contrib;
+                    os_k[j][k] = has[j] ? a.os[col * RANK + k] : 0.0f;
+                    S[j] = S[j] + vs_k[k] * os_k[j][k];
                 }
-                // the tile row's 4 dx terms, summed on the quad, into the
-                // block row's LDS row (4 tiles of a pass add to one address)
-                const float qdx = quad_sum(tdx);
-                if (lj == 0u && tile_ok) atomicAdd(&sdx[(int64_t)li * B + b], qdx);
-                // a quad is one tile row: full is uniform over it
+                q0[j] = fp4_decode(byte & 0xFu);
+                s.q[j] = q0[j];
+                s.ci[j] = fp4_decode(byte >> 4) * (imp_scale * ((a.ois && has[j]) ? a.ois[col] : 1.0f));
+                ok = ok && (!has[j] || scale_in_range(S[j]));
+            }
+#pragma unroll
+            for (int k = 0; k < 2 * RANK; ++k) s.mr[k] = 0.0;
+#pragma unroll
+            for (int j = 0; j < (COLS ? 4 : 1); ++j)
+#pragma unroll
+                for (int k = 0; k < 2 * RANK; ++k) s.mc[j][k] = 0.0f;
+            const bool lane_on = tile_ok && row_ok;
+            // lanes without a tile row (past the row's last tile, rows past
+            // n_in) step zeros; a wave holding an edge tile steps as written
+            const bool fast = a.fast && __all(!lane_on || (full && ok));
+            // one batch step of the lane's 4 slots (b in order), as written:
+            // the sum of their dx terms
+            auto exact_step = [&](int64_t b) -> float {
+                const float iv = xl[b];
+                float u[RANK][4], v[RANK][4], dx = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float dyv = has[j] ? g0[j * B + b] : 0.0f;
+                    const float g = dyv * iv, contrib = q0[j] * iv;
+                    s.ci[j] = bounded_update_ci(s.ci[j], g, contrib, a.beta2, a.min_decay_frac, a.max_ci);
+                    s.q[j] = s.q[j] + bounded_update_cw(g, s.ci[j], S[j], eff_lr, a.eps, a.damp != 0, a.max_abs_delta);
+                    const float qf = (s.q[j] == 0.0f) ? a.zero_escape_eps : s.q[j];
+                    dx = dx + (has[j] ? (s.q[j] * S[j]) * dyv : 0.0f);
+#pragma unroll
+                    for (int k = 0; k < RANK; ++k) {
+                        if constexpr (COLS) {
+                            s.mc[j][k] = s.mc[j][k] + (qf * vs_k[k]) * g;
+                            s.mc[j][RANK + k] = s.mc[j][RANK + k] + (qf * vs_k[k]) * contrib;
+                        }
+                        if (full) {
+                            u[k][j] = (qf * os_k[j][k]) * g;
+                            v[k][j] = (qf * os_k[j][k]) * contrib;
+                        } else if (has[j]) {
+                            s.mr[k] = s.mr[k] + ((double)qf * (double)os_k[j][k]) * (double)g;
+                            s.mr[RANK + k] = s.mr[RANK + k] + ((double)qf * (double)os_k[j][k]) * (double)contrib;
+                        }
+                    }
+                }
                 if (full) {
 #pragma unroll
                     for (int k = 0; k < RANK; ++k) {
-                        mr[k] = mr[k] + (double)quad_sum((qf * os_k[k]) * g);
-                        mr[RANK + k] = mr[RANK + k] + (double)quad_sum((qf * os_k[k]) * contrib);
+                        s.mr[k] = s.mr[k] + (double)(((u[k][0] + u[k][1]) + u[k][2]) + u[k][3]);
+                        s.mr[RANK + k] = s.mr[RANK + k] + (double)(((v[k][0] + v[k][1]) + v[k][2]) + v[k][3]);
                     }
-                } else {
+                }
+                return dx;
+            };
+            auto fast_step = [&](float iv, const float (&dy)[4], StepRange &rg) -> float {
+                float u[RANK][4], v[RANK][4], dx = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float g = dy[j] * iv, contrib = q0[j] * iv;
+                    fast_update(s.ci[j], s.q[j], g, contrib, S[j], eff_lr, a.beta2, omb, a.eps, a.max_ci,
+                                a.max_abs_delta, rg);
+                    const float qf = (s.q[j] == 0.0f) ? a.zero_escape_eps : s.q[j];
+                    dx = __builtin_fmaf(s.q[j] * S[j], dy[j], dx);
 #pragma unroll
                     for (int k = 0; k < RANK; ++k) {
-                        const double d0 = has ? ((double)qf * (double)os_k[k]) * (double)g : 0.0;
-                        const double d1 = has ? ((double)qf * (double)os_k[k]) * (double)contrib : 0.0;
-                        mr[k] = (((mr[k] + quad_lane<0>(d0)) + quad_lane<1>(d0)) + quad_lane<2>(d0)) + quad_lane<3>(d0);
-                        mr[RANK + k] =
-                            (((mr[RANK + k] + quad_lane<0>(d1)) + quad_lane<1>(d1)) + quad_lane<2>(d1)) + quad_lane<3>(d1);
+                        if constexpr (COLS) {
+                            s.mc[j][k] = s.mc[j][k] + (qf * vs_k[k]) * g;
+                            s.mc[j][RANK + k] = s.mc[j][RANK + k] + (qf * vs_k[k]) * contrib;
+                            pin_here(s.mc[j][k]);
+                            pin_here(s.mc[j][RANK + k]);
+                        }
+                        u[k][j] = (qf * os_k[j][k]) * g;
+                        v[k][j] = (qf * os_k[j][k]) * contrib;
                     }
                 }
+#pragma unroll
+                for (int k = 0; k < RANK; ++k) {
+                    s.mr[k] = s.mr[k] + (double)(((u[k][0] + u[k][1]) + u[k][2]) + u[k][3]);
+                    s.mr[RANK + k] = s.mr[RANK + k] + (double)(((v[k][0] + v[k][1]) + v[k][2]) + v[k][3]);
+                    pin_here(s.mr[k]);
+                    pin_here(s.mr[RANK + k]);
+                }
+                return dx;
+            };
+            // the lanes' dx terms of steps b..b+3: summed over the 4 tiles of
+            // each DPP row; lane (tile t, li) of it then adds step b + t of row li
+            auto add_dx = [&](int64_t b, float (&d)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    d[i] += dpp_f32<DPP_ROW_ROR4>(d[i]);
+                    d[i] += dpp_f32<DPP_ROW_ROR8>(d[i]);
+                }
+                const uint32_t i = tl & 3u;
+                const float v = i == 0u ? d[0] : i == 1u ? d[1] : i == 2u ? d[2] : d[3];
+                atomicAdd(&sdx[(int64_t)li * LD + b + i], v);
             };
             int64_t b = 0;
-            if ((B & 3) == 0) {
-                // 4 batch steps per pair of 16-byte loads (rows are B floats, B % 4 == 0)
-                for (; b < B; b += 4) {
-                    const float4 xv = *reinterpret_cast<const float4 *>(xrow + b);
-                    const float4 gv = *reinterpret_cast<const float4 *>(gcol + b);
-                    step(b, xv.x, gv.x);
-                    step(b + 1, xv.y, gv.y);
-                    step(b + 2, xv.z, gv.z);
-                    step(b + 3, xv.w, gv.w);
+            float4 nx[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                nx[j] = fast && B >= 4 ? load_f4(g0 + j * B) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (; b + 4 <= B; b += 4) {
+                float dx4[4];
+                bool done = false;
+                if (fast) {
+                    const B4State<RANK, COLS> keep = s;
+                    const float4 xv = *reinterpret_cast<const float4 *>(xl + b);
+                    const float x[4] = {xv.x, xv.y, xv.z, xv.w};
+                    float dy[4][4];  // [step][slot]
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        dy[0][j] = nx[j].x;
+                        dy[1][j] = nx[j].y;
+                        dy[2][j] = nx[j].z;
+                        dy[3][j] = nx[j].w;
+                        if (b + 8 <= B) nx[j] = load_f4(g0 + j * B + b + 4);
+                    }
+                    StepRange rg;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        dx4[i] = fast_step(x[i], dy[i], rg);
+                        // the 4 slots' chains interleave; interleaving steps too
+                        // only costs registers (spills at 4 waves per SIMD)
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    done = !__any(lane_on && rg.outside());
+                    if (!done) s = keep;
                 }
+                if (!done) {
+#pragma unroll 1
+                    for (int i = 0; i < 4; ++i) {
+                        const float d = exact_step(b + i);
+                        dx4[0] = i == 0 ? d : dx4[0];
+                        dx4[1] = i == 1 ? d : dx4[1];
+                        dx4[2] = i == 2 ? d : dx4[2];
+                        dx4[3] = i == 3 ? d : dx4[3];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dx4[i] = lane_on ? dx4[i] : 0.0f;
+                add_dx(b, dx4);
             }
-            for (; b < B; ++b) step(b, xrow[b], gcol[b]);
-            if (has) {
-                const float imp = ci / cis;
+            if (b < B) {  // the last 1..3 steps (LDS rows hold b4_ld(B) > B + 3 floats)
+                float dx4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (int64_t i = 0; b + i < B; ++i) {
+                    const float d = exact_step(b + i);
+                    dx4[0] = i == 0 ? d : dx4[0];
+                    dx4[1] = i == 1 ? d : dx4[1];
+                    dx4[2] = i == 2 ? d : dx4[2];
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) dx4[i] = lane_on ? dx4[i] : 0.0f;
+                add_dx(b, dx4);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (!has[j]) continue;
+                const uint32_t slot = (uint32_t)j * 4u + li;
+                const float imp = s.ci[j] / (imp_scale * (a.ois ? a.ois[c0 + j] : 1.0f));
                 uint32_t wq, iq;
                 if (a.stochastic) {
-                    const uint64_t base = a.seed + 2ull * (uint64_t)(a.nnz_scattered + t * 16 + slot);
-                    wq = fp4_encode_stochastic(q, splitmix64(base));
+                    const uint64_t base = a.seed + 2ull * ((uint64_t)a.nnz_scattered + (uint64_t)t * 16 + slot);
+                    wq = fp4_encode_stochastic(s.q[j], splitmix64(base));
                     iq = fp4_encode_stochastic(imp, splitmix64(base + 1ull));
                 } else {
-                    wq = fp4_encode(q);
+                    wq = fp4_encode(s.q[j]);
                     iq = fp4_encode(imp);
                 }
-                a.tiles[t * 16 + slot] = (uint8_t)((iq << 4) | wq);
-                if (a.b4term) {
+                a.tiles[(uint64_t)t * 16 + slot] = (uint8_t)((iq << 4) | wq);
+                if constexpr (COLS) {
 #pragma unroll
-                    for (int k = 0; k < 2 * RANK; ++k) a.b4term[(t * 16 + slot) * 2 * RANK + k] = mc[k];
+                    for (int k = 0; k < 2 * RANK; ++k) a.b4term[((uint64_t)t * 16 + slot) * 2 * RANK + k] = s.mc[j][k];
                 }
             }
-            // the tile rows' fp64 partials, added per row in tile order
-            if (lj == 0u) {
 #pragma unroll
-                for (int k = 0; k < 2 * RANK; ++k) s_mr[wave][tl][li][k] = tile_ok ? mr[k] : 0.0;
-            }
-            wave_lds_sync();
-            if (lane < 4u) {
-                for (uint32_t u = 0; u < 4u && sub + u < nt; ++u) {
-#pragma unroll
-                    for (int k = 0; k < 2 * RANK; ++k) rowacc[k] = rowacc[k] + s_mr[wave][u][lane][k];
-                }
-            }
-            wave_lds_sync();
+            for (int k = 0; k < 2 * RANK; ++k) s_mr[wave * 16u + tl][li][k] = s.mr[k];
         }
-        carry = chunk_advance(ch, pos, ebase);
+        __syncthreads();
+        // the tile rows' fp64 partials, added per row in tile order
+        if (threadIdx.x < 8u * RANK) {
+            const uint32_t l = threadIdx.x / (2u * RANK), k = threadIdx.x % (2u * RANK);
+            const uint32_t n = min(TILES_B4, t1 - p0);
+            double sum = s_row[l][k];
+            for (uint32_t u = 0; u < n; ++u) sum = sum + s_mr[u][l][k];
+            s_row[l][k] = sum;
+        }
+        __syncthreads();
     }
-    wave_lds_sync();
-    for (uint32_t l = 0; l < 4u; ++l) {
-        const int64_t rr = br * 4 + l;
-        if (rr >= a.n_in) break;
-        for (int64_t b = lane; b < B; b += 64) a.dx[b * a.n_in + rr] += sdx[(int64_t)l * B + b];
+    for (int64_t i = threadIdx.x; i < 4 * B; i += 256) {
+        const int64_t l = i & 3, b = i >> 2, rr = br * 4 + l;
+        if (rr >= a.n_in) continue;
+        float v = 0.0f;
+#pragma unroll
+        for (uint32_t w = 0; w < WAVES_B4; ++w) v += s_dyn[((1 + w) * 4 + l) * LD + b];
+        a.dx[b * a.n_in + rr] += v;
     }
     // the block rows' scale step (linear_disldo.hpp:1923-1951)
-    const int64_t r = br * 4 + lane;
-    if (lane < 4u && r < a.n_in) {
+    const int64_t r = br * 4 + threadIdx.x;
+    if (threadIdx.x < 4u && r < a.n_in) {
         const float scale_eff_lr = a.lr / (float)nnz_row;
 #pragma unroll
         for (int k = 0; k < RANK; ++k) {
-            const double sum = rowacc[k], sum_c = rowacc[RANK + k];
+            const double sum = s_row[threadIdx.x][k], sum_c = s_row[threadIdx.x][RANK + k];
             if (sum == 0.0 && sum_c == 0.0) continue;
             const float g_agg = (float)sum, contrib_agg = (float)sum_c;
             if (!finite_f(g_agg) || !finite_f(contrib_agg)) continue;
@@ -1194,6 +1461,19 @@ void launch_rows_kernel(int rank, bool deferred, bool cols, dim3 grid, dim3 bloc
     }
 }
 
+template <int RANK>
+void launch_b4_rank(const B4TrainArgs &a, hipStream_t st) {
+    // x and each wave's dx rows: up to 82 KB at batch 1024
+    const uint32_t lds = (uint32_t)((1 + WAVES_B4) * 4 * b4_ld(a.B) * sizeof(float));
+    auto go = [&](auto kernel) {
+        SILI_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)lds));
+        launch(kernel, dim3((unsigned)a.brows), dim3(64 * WAVES_B4), lds, st, a);
+    };
+    if (a.b4term) go(&k_train_b4<RANK, true>);
+    else go(&k_train_b4<RANK, false>);
+}
+
 }  // namespace
 
 void launch_train_rows(Layer &L, const float *xT, const float *gT, int64_t B, float *dx, const TrainParams &p,
@@ -1242,9 +1522,10 @@ void launch_train_rows(Layer &L, const float *xT, const float *gT, int64_t B, fl
     a.lr_per_row_nnz = p.lr_per_row_nnz;
     a.damp = p.damp_by_importance;
     a.stochastic = L.stochastic_rounding ? 1 : 0;
+    a.fast = fast_step_params(p) ? 1 : 0;
     a.seed = seed;
     const dim3 grid((unsigned)((L.n_in + WAVES_T - 1) / WAVES_T)), block(256);
-    const uint32_t lds = (uint32_t)(WAVES_T * (2 * B + 512) * sizeof(float));
+    const uint32_t lds = (uint32_t)(WAVES_T * (2 * ((B + 3) & ~(int64_t)3) + 512) * sizeof(float));
     ProfScope ps("train_rows", st);
     launch_rows_kernel(L.rank, a.deferred != 0, a.mterm != nullptr, grid, block, lds, st, a);
     SILI_HIP(hipGetLastError());
@@ -1276,7 +1557,7 @@ void launch_sparse_train(Layer &L, const float *xT, const float *gT, int64_t B, 
     a.damp = p.damp_by_importance;
     ProfScope ps("sparse_train_rows", st);
     launch(k_sparse_train_rows, dim3((unsigned)((L.n_in + WAVES_T - 1) / WAVES_T)), dim3(256),
-           (uint32_t)(WAVES_T * (2 * B + 512) * sizeof(float)), st, a);
+           (uint32_t)(WAVES_T * (2 * ((B + 3) & ~(int64_t)3) + 512) * sizeof(float)), st, a);
     launch(k_sparse_train_vs, dim3(nblk(L.n_in)), dim3(TPB), 0, st, (const uint32_t *)L.W.elem_start.p, L.n_in,
            L.rank, (const double *)L.train_rowsum.p, L.vs.p, L.vs_imp.p, L.vs_step.p, p.lr, p.beta2, p.eps,
            (const float *)L.pow_tab.p);
@@ -1341,9 +1622,8 @@ void launch_train_b4(Layer &L, const float *xT, const float *gT, int64_t B, floa
                      uint64_t seed, hipStream_t st) {
     if (L.B4.ntiles == 0) return;
     B4TrainArgs a{};
-    a.byte_start = L.B4.byte_start.p;
     a.tile_start = L.B4.tile_start.p;
-    a.idx = L.B4.idx.p;
+    a.tcol = b4_tile_cols(L);
     a.tiles = L.B4.tiles.p;
     a.brows = L.B4.brows;
     a.n_in = L.n_in;
@@ -1374,15 +1654,14 @@ void launch_train_b4(Layer &L, const float *xT, const float *gT, int64_t B, floa
     a.lr_per_row_nnz = p.lr_per_row_nnz;
     a.damp = p.damp_by_importance;
     a.stochastic = L.stochastic_rounding ? 1 : 0;
+    a.fast = fast_step_params(p) ? 1 : 0;
     a.seed = seed;
-    const dim3 grid((unsigned)((L.B4.brows + WAVES_B4 - 1) / WAVES_B4)), block(64 * WAVES_B4);
-    const uint32_t shmem = (uint32_t)(WAVES_B4 * 4 * B * sizeof(float));  // B <= 1024: <= 32 KiB
     ProfScope ps("train_b4", st);
     switch (L.rank) {
-        case 1: launch(k_train_b4<1>, grid, block, shmem, st, a); break;
-        case 2: launch(k_train_b4<2>, grid, block, shmem, st, a); break;
-        case 3: launch(k_train_b4<3>, grid, block, shmem, st, a); break;
-        default: launch(k_train_b4<4>, grid, block, shmem, st, a); break;
+        case 1: launch_b4_rank<1>(a, st); break;
+        case 2: launch_b4_rank<2>(a, st); break;
+        case 3: launch_b4_rank<3>(a, st); break;
+        default: launch_b4_rank<4>(a, st); break;
     }
     SILI_HIP(hipGetLastError());
 }
