@@ -208,16 +208,6 @@ __device__ __forceinline__ void fast_update(float &ci, float &wv, float g, float
     wv = wv + eff_lr * __builtin_amdgcn_fmed3f(raw, -max_abs_delta, max_abs_delta);
 }
 
-// 16-byte load from an address that is 4-byte aligned (a feature-major row of
-// a batch that is no multiple of 4).
-__device__ __forceinline__ float4 load_f4(const float *p) {
-    struct __attribute__((packed, aligned(4))) F4 {
-        float x, y, z, w;
-    };
-    const F4 v = *reinterpret_cast<const F4 *>(p);
-    return make_float4(v.x, v.y, v.z, v.w);
-}
-
 // The lanes' 8 terms of batch steps b0..b0+7 (lane l's in sred[8 l ..])
 // summed over the lanes into rdx[b0..b0+n): each lane adds one step's values
 // of 8 lanes (read in a rotated order so that the wave's 64 reads hit 64
@@ -716,12 +706,14 @@ struct B4TrainArgs {
 // tile, whose 4 columns are not all in range, adds its fp64 row-gradient terms
 // one by one (the reference's scalar path).  The tiles' fp64 row partials are
 // added in tile order; then the block rows' scale step.  dx: per 4 batch steps
-// the lanes' sums of a DPP row's 4 tiles go to the wave's own LDS rows by one
-// add per lane; the waves' rows are added in wave order at the end.
+// the tile rows' sums turn in LDS and 16 lanes add them in tile order, as the
+// reference does (an LDS float add with several lanes per address took 150
+// clocks a wave); the waves' rows are added in wave order at the end.
 constexpr uint32_t WAVES_B4 = 4;  // waves per block of k_train_b4
 constexpr uint32_t TILES_B4 = 16 * WAVES_B4;  // tiles the block takes at a time
 // Floats of a row of batch values in LDS: 16-byte aligned, and 4 more so that
 // the 4 rows' reads of one step group fall into different banks.
+constexpr uint32_t TURN_LD = 20;  // a (row, step)'s 16 tiles in LDS, 16-byte aligned
 __host__ __device__ inline int64_t b4_ld(int64_t B) { return ((B + 3) & ~(int64_t)3) + 4; }
 
 // A lane's state while its 4 slots train.
@@ -736,13 +728,14 @@ template <int RANK, bool COLS>
 __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4TrainArgs a) {
     __shared__ double s_mr[TILES_B4][4][2 * RANK];  // [tile][li][k | contrib k]
     __shared__ double s_row[4][2 * RANK];           // the rows' sums over all tiles
+    __shared__ __attribute__((aligned(16))) float s_turn[WAVES_B4][16 * TURN_LD];
     extern __shared__ __attribute__((aligned(16))) float s_dyn[];  // x [4][LD], then dx [wave][4][LD]
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const int64_t br = blockIdx.x;
     const uint32_t t0 = a.tile_start[br], t1 = a.tile_start[br + 1];
     if (t0 == t1) return;  // the whole block
     const int64_t B = a.B, LD = b4_ld(B);
-    float *sx = s_dyn, *sdx = s_dyn + (1 + wave) * 4 * LD;
+    float *sx = s_dyn, *sdx = s_dyn + (1 + wave) * 4 * LD, *sturn = s_turn[wave];
     for (int64_t i = threadIdx.x; i < 4 * LD; i += 256) {
         const int64_t l = i / LD, b = i % LD;
         sx[i] = b < B && br * 4 + l < a.n_in ? a.xT[(br * 4 + l) * B + b] : 0.0f;
@@ -845,7 +838,7 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
                     fast_update(s.ci[j], s.q[j], g, contrib, S[j], eff_lr, a.beta2, omb, a.eps, a.max_ci,
                                 a.max_abs_delta, rg);
                     const float qf = (s.q[j] == 0.0f) ? a.zero_escape_eps : s.q[j];
-                    dx = __builtin_fmaf(s.q[j] * S[j], dy[j], dx);
+                    dx = dx + (s.q[j] * S[j]) * dy[j];
 #pragma unroll
                     for (int k = 0; k < RANK; ++k) {
                         if constexpr (COLS) {
@@ -867,17 +860,27 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
                 }
                 return dx;
             };
-            // the lanes' dx terms of steps b..b+3: summed over the 4 tiles of
-            // each DPP row; lane (tile t, li) of it then adds step b + t of row li
-            auto add_dx = [&](int64_t b, float (&d)[4]) {
+            // the lanes' dx terms of steps b..b+3: turned in LDS, lane (li,
+            // step) then adds the wave's 16 tiles in tile order
+            auto add_dx = [&](int64_t b, const float (&d)[4]) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    d[i] += dpp_f32<DPP_ROW_ROR4>(d[i]);
-                    d[i] += dpp_f32<DPP_ROW_ROR8>(d[i]);
+                for (int i = 0; i < 4; ++i) sturn[(li * 4u + (uint32_t)i) * TURN_LD + tl] = d[i];
+                wave_lds_sync();
+                if (lane < 16u) {
+                    float *to = &sdx[(int64_t)(lane >> 2) * LD + b + (lane & 3u)];
+                    const float4 *from = reinterpret_cast<const float4 *>(sturn + lane * TURN_LD);
+                    float v = *to;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float4 f = from[u];
+                        v = v + f.x;
+                        v = v + f.y;
+                        v = v + f.z;
+                        v = v + f.w;
+                    }
+                    *to = v;
                 }
-                const uint32_t i = tl & 3u;
-                const float v = i == 0u ? d[0] : i == 1u ? d[1] : i == 2u ? d[2] : d[3];
-                atomicAdd(&sdx[(int64_t)li * LD + b + i], v);
+                wave_lds_sync();
             };
             int64_t b = 0;
             float4 nx[4];

@@ -242,6 +242,22 @@ __device__ __forceinline__ float4 buffer_load_f4(__amdgpu_buffer_rsrc_t r, uint3
 __device__ __forceinline__ float buffer_load_f1(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
 }
+// 16-byte load from an address that is 4-byte aligned (a feature-major row of
+// a batch that is no multiple of 4).
+__device__ __forceinline__ float4 load_f4(const float *p) {
+    struct __attribute__((packed, aligned(4))) F4 {
+        float x, y, z, w;
+    };
+    const F4 v = *reinterpret_cast<const F4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float2 load_f2(const float *p) {
+    struct __attribute__((packed, aligned(4))) F2 {
+        float x, y;
+    };
+    const F2 v = *reinterpret_cast<const F2 *>(p);
+    return make_float2(v.x, v.y);
+}
 // An offset no buffer used here reaches: loads from it return 0.
 constexpr uint32_t OOB_OFFSET = 0x80000000u;
 
