@@ -835,6 +835,8 @@ void build_scattered(Layer &L, DScatter &dst, int64_t rows, int64_t ncols, int64
     dst.sh_valid = false;
     dst.n_short_hint = e.n_short;
     dst.slc_w = 0;
+    dst.drop_m24();
+    dst.m24_failed = false;
     dst.stream1.failed = dst.streamK.failed = false;
     dst.cblk.clear();
     dst.cblk_cb = 0;
@@ -898,6 +900,8 @@ void build_shadow(Layer &L, const DScatter &src, const uint32_t *d_rows, const u
     dst.sh_valid = false;
     dst.n_short_hint = e.n_short;
     dst.slc_w = 0;
+    dst.drop_m24();
+    dst.m24_failed = false;
     dst.cblk.clear();
     dst.cblk_cb = 0;
     dst.rows = src.cols;

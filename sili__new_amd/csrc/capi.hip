@@ -478,24 +478,28 @@ void forward_dense(Layer &L, const float *x, int64_t B, float *y, hipStream_t st
     ProfCtx pc(L, "fwd");
     if (B <= 0) throw_error(SILI_ERR_INVALID, "forward_dense: batch must be >= 1");
     if (!x || !y) throw_error(SILI_ERR_INVALID, "forward_dense: NULL buffer");
-    // the input's feature-major copy and the output's zeroing in one launch
-    Prep prep(st);
-    const float *xT = prep.feature_major(L.ws_xT, x, B, L.n_in, nullptr);
-    // the feature-major copy doubles as the stored forward input that
-    // backward_dense reads when called without x (sili/cpu_backend.cpp:481)
-    L.xT_cached_batch = B > 1 ? B : 0;
     // scattered pass skips exact-zero inputs (linear_disldo.hpp:114); only
     // observable with non-finite weights, so the skip is compiled in only then
     const int skip = L.has_nonfinite ? SKIP_ZERO : SKIP_NONE;
     const ScaleView ssc = shadow_scales(L);
-    const bool str = L.Wt.nnz > 0 && stream_wanted(L.Wt, ssc, B, B, skip);
+    const bool m24 = mfma24_wanted(L, L.Wt, ssc, B, skip, st);
+    // the input's feature-major copy and the output's zeroing in one launch
+    // (the matrix-core gather makes the copy beside its operands)
+    Prep prep(st);
+    if (m24) L.ws_xT.ensure((size_t)(L.n_in * B));
+    const float *xT = m24 ? L.ws_xT.p : prep.feature_major(L.ws_xT, x, B, L.n_in, nullptr);
+    // the feature-major copy doubles as the stored forward input that
+    // backward_dense reads when called without x (sili/cpu_backend.cpp:481)
+    L.xT_cached_batch = B > 1 ? B : 0;
+    const bool str = L.Wt.nnz > 0 && !m24 && stream_wanted(L.Wt, ssc, B, B, skip);
     // batches 65..128: the input staged in LDS slice by slice (SILI_STAGED)
-    const bool staged = L.Wt.nnz > 0 && !str && env_int("SILI_STAGED", 1) && staged_supported(L, L.Wt, ssc, xT, B, skip);
-    const bool plain = L.Wt.nnz > 0 && !str && !staged && colblock_passes(L.Wt, xT, B) == 0;
+    const bool staged = L.Wt.nnz > 0 && !m24 && !str && env_int("SILI_STAGED", 1) && staged_supported(L, L.Wt, ssc, xT, B, skip);
+    const bool plain = L.Wt.nnz > 0 && !m24 && !str && !staged && colblock_passes(L.Wt, xT, B) == 0;
     if (L.Wt.nnz == 0) prep.fill(y, B * L.n_out, 0.0f);
     else if (plain) prep.zero_split(L.Wt.plan(), y, L.n_out, B);
     prep.run();
-    if (str) stream_gather(L, L.Wt, ssc, xT, B, y, L.n_out, st);
+    if (m24) launch_mfma24(L, L.Wt, ssc, x, L.n_in, xT, L.ws_xT.p, B, y, L.n_out, st);
+    else if (str) stream_gather(L, L.Wt, ssc, xT, B, y, L.n_out, st);
     else if (staged) launch_gather_staged(L, L.Wt, ssc, xT, B, y, L.n_out, st);
     else if (plain) launch_gather(gather_plan(L, L.Wt, B), ssc, xT, B, y, L.n_out, B, skip, st);
     else if (L.Wt.nnz > 0 && !gather_colblocked(L, L.Wt, ssc, xT, B, y, L.n_out, skip, st))
@@ -582,13 +586,15 @@ void backward_dense(Layer &L, const float *x, const float *dy, int64_t B, float 
     // grad-input and grad-W read the same gT row per synapse: one fused pass
     // when grad-W is wanted; otherwise the stream kernels (small batches) or
     // the segment gather
-    const bool str = scat && !gw_s && stream_wanted(L.W, canon_scales(L), B, B, SKIP_NONE);
+    const bool m24 = scat && !gw_s && mfma24_wanted(L, L.W, canon_scales(L), B, SKIP_NONE, st);
+    const bool str = scat && !gw_s && !m24 && stream_wanted(L.W, canon_scales(L), B, B, SKIP_NONE);
     if (!scat) prep.fill(dx, B * L.n_in, 0.0f);
-    else if (!str) prep.zero_split(L.W.plan(), dx, L.n_in, B);
+    else if (!str && !m24) prep.zero_split(L.W.plan(), dx, L.n_in, B);
     prep.run();
     const bool fused = scat && gw_s &&
                        launch_bwd_fused(L.W.plan(), canon_scales(L), gT, xT, B, dx, L.n_in, gw_s, L.acc_in.p, st);
-    if (str) stream_gather(L, L.W, canon_scales(L), gT, B, dx, L.n_in, st);
+    if (m24) launch_mfma24(L, L.W, canon_scales(L), dy, L.n_out, gT, nullptr, B, dx, L.n_in, st);
+    else if (str) stream_gather(L, L.W, canon_scales(L), gT, B, dx, L.n_in, st);
     else if (scat && !fused && !gather_colblocked(L, L.W, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st))
         launch_gather(gather_plan(L, L.W, B), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
     if (L.B4.ntiles > 0 && !gather_b4_colblocked(L, L.B4, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st))
@@ -691,6 +697,7 @@ void backward_dense_train(Layer &L, const float *x, const float *dy, int64_t B, 
     // copies holding value bytes are stale now: rebuilt on their next use
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
+        sc->drop_m24();
         sc->cblk.clear();
         sc->cblk_cb = 0;
     }
@@ -781,6 +788,7 @@ void backward_sparse_train(Layer &L, const float *x, const int32_t *dptrs, const
     launch_b4_shadow_refresh(L, st);
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
+        sc->drop_m24();
         sc->cblk.clear();
         sc->cblk_cb = 0;
     }

@@ -117,6 +117,24 @@ struct DScatter {
     DevBuf<uint8_t> slc_col;
     DevBuf<uint32_t> slc_off;
     int64_t slc_w = 0, slc_n = 0;
+    // the 2:4 copy of the matrix-core gather (mfma24.hip; built on first use,
+    // dropped when values or structure change): FP4 codes and positions per 32
+    // rows x 128 columns, and the entries that a group of 4 columns has no
+    // place for, by row
+    DevBuf<uint4> m24_val;
+    DevBuf<uint2> m24_idx;
+    DevBuf<uint32_t> m24_ovf_start;
+    DevBuf<uint2> m24_ovf;
+    bool m24_valid = false, m24_failed = false;
+    uint32_t m24_n_ovf = 0, m24_max_ovf = 0;  // overflow entries: all, and the most of a row
+    // us it saved or would have saved since the values last changed, and when
+    // to build it: m24_saved >= m24_cost * m24_wait
+    double m24_saved = 0, m24_cost = 0, m24_wait = 1;
+    void drop_m24() {
+        if (m24_valid) m24_wait = m24_saved < m24_cost * (m24_wait + 1) ? std::min(m24_wait * 2, 1e6) : 1;
+        m24_valid = false;
+        m24_saved = 0;
+    }
     // column-block copies for gathers whose operand exceeds one XCD's L2:
     // cblk[k] holds every row's entries with columns in [k*cblk_cb, ...),
     // columns relative to the block (built on first use)
@@ -365,6 +383,9 @@ struct Layer {
     DevBuf<float> ws_xT, ws_gT, ws_out;
     DevBuf<float> ws_s0;  // component 0 of rank > 1 scales: value [n_in], then output [n_out]
     DevBuf<float> ws_xs;  // the staged-input gather's column-scaled input copy
+    DevBuf<uint16_t> ws_m24;  // the matrix-core gather's input pieces (bf16)
+    DevBuf<int> m24_flag;     // set by its split kernel to the call's number: an input has no pieces
+    int m24_epoch = 0;
     int64_t xT_cached_batch = 0;  // > 0: ws_xT holds the last forward_dense input, feature-major
     Scratch scratch;
     Profiler prof;
@@ -657,6 +678,12 @@ void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb);
 bool staged_supported(const Layer &L, const DScatter &s, const ScaleView &sc, const float *in, int64_t B, int skip);
 void launch_gather_staged(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t B, float *out,
                           int64_t out_ld, hipStream_t st);
+// The matrix-core gather (mfma24.hip): whether it takes this case (its copy of
+// the store is then built), and out[b, r] for every row r of s (written).  in: batch-major [B][in_ld], inT: the same feature-major, which
+// the call itself fills when xT == inT is given (NULL: filled before).
+bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int skip, hipStream_t st);
+void launch_mfma24(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t in_ld, const float *inT,
+                   float *xT, int64_t B, float *out, int64_t out_ld, hipStream_t st);
 // b.rng_* for K column ranges of ceil(bcols / K) block columns.
 void ensure_col_ranges(Layer &L, DBlock4 &b, int K);
 // Block4 contribution (added into out) in column-block passes when the

@@ -119,6 +119,7 @@ void requantize_code8(Layer &L) {
     // copies holding value bytes are stale: rebuilt on their next use
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
+        sc->drop_m24();
         sc->cblk.clear();
         sc->cblk_cb = 0;
     }

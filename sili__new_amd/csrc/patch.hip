@@ -682,6 +682,8 @@ void invalidate_derived(DScatter &s) {
     s.dcol_valid = false;
     s.sh_valid = false;
     s.slc_w = 0;
+    s.drop_m24();
+    s.m24_failed = false;
     s.cblk.clear();
     s.cblk_cb = 0;
 }
