@@ -812,7 +812,7 @@ void ensure_short_rows(Layer &L, DScatter &s) {
 
 GatherPlan gather_plan(Layer &L, DScatter &s, int64_t nb) {
     GatherPlan p = s.plan();
-    if (nb > 1 && nb <= SHORT_MAX_BATCH && nb % 4 == 0) {
+    if (nb > 1 && nb <= SHORT_MAX_BATCH) {
         ensure_short_rows(L, s);
         if (s.n_sh > 0) {
             p.sh_seg = s.sh_seg.p;

@@ -22,7 +22,7 @@ struct sili_layer {
 // The no-allocation forward's scratch: every GPU the library runs on holds its
 // own copy until the process ends.
 constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(32) << 20;
-static __device__ __align__(256) float scratch[NOALLOC_SCRATCH_BYTES / sizeof(float)];
+static __device__ __align__(256) float scratch[NOALLOC_SCRATCH_BYTES / sizeof(float) + sili::BATCH_SLACK];
 
 namespace sili {
 
@@ -351,7 +351,7 @@ const float *to_feature_major(Layer &L, DevBuf<float> &ws, const float *x, int64
         if (acc) launch_colabs(x, 1, n, acc, st);
         return x;
     }
-    ws.ensure((size_t)(n * B));
+    ws.ensure((size_t)(n * B + BATCH_SLACK));
     launch_transpose(x, B, n, ws.p, acc, st);
     return ws.p;
 }
@@ -378,7 +378,7 @@ struct Prep {
             if (acc) colabs(x, 1, cols, acc);
             return x;
         }
-        ws.ensure((size_t)(cols * B));
+        ws.ensure((size_t)(cols * B + BATCH_SLACK));
         if (room() && B % 4 == 0 && cols % 4 == 0 && al16(x) && al16(ws.p)) add(PREP_TRANSPOSE, x, ws.p, acc, B, cols);
         else launch_transpose(x, B, cols, ws.p, acc, st);
         return ws.p;
@@ -422,7 +422,7 @@ struct Prep {
 // 2 MiB beat 4 of 4 MiB and 2 of 8 MiB).
 int64_t colblock_passes(const DScatter &s, const float *in, int64_t B) {
     const int mode = env_int("SILI_COLBLOCK", 1);
-    if (mode == 0 || s.nnz == 0 || B % 4 != 0 || B > 512 || (reinterpret_cast<uintptr_t>(in) & 15u) != 0) return 0;
+    if (mode == 0 || s.nnz == 0 || B < 2 || B > 512) return 0;
     const int64_t opbytes = s.cols * B * 4;
     if (opbytes <= (int64_t(4) << 20) || opbytes >= (int64_t)0x80000000LL) return 0;
     const int64_t slice = (int64_t)std::max(1, env_int("SILI_COLBLOCK_MB", 2)) << 20;
@@ -486,7 +486,7 @@ void forward_dense(Layer &L, const float *x, int64_t B, float *y, hipStream_t st
     // the input's feature-major copy and the output's zeroing in one launch
     // (the matrix-core gather makes the copy beside its operands)
     Prep prep(st);
-    if (m24) L.ws_xT.ensure((size_t)(L.n_in * B));
+    if (m24) L.ws_xT.ensure((size_t)(L.n_in * B + BATCH_SLACK));
     const float *xT = m24 ? L.ws_xT.p : prep.feature_major(L.ws_xT, x, B, L.n_in, nullptr);
     // the feature-major copy doubles as the stored forward input that
     // backward_dense reads when called without x (sili/cpu_backend.cpp:481)
@@ -729,7 +729,7 @@ void forward_sparse(Layer &L, const int32_t *ptrs, const int32_t *idx, const flo
     const bool push = push_supported(L) && push_mode != 0 && (push_mode == 2 || sparse_enough);
     if (push) launch_push_fwd(L, ptrs, idx, vals, B, comp0_scales(L, false, st), y, false, st);
     if (!push || L.B4t.ntiles > 0) {
-        L.ws_xT.ensure((size_t)(L.n_in * B));
+        L.ws_xT.ensure((size_t)(L.n_in * B + BATCH_SLACK));
         launch_densify_full(ptrs, idx, vals, B, L.n_in, L.ws_xT.p, nullptr, true, nnz_x, st);
     }
     const ScaleView ssc = comp0_scales(L, true, st);
@@ -746,7 +746,7 @@ void backward_sparse(Layer &L, const float *x, const int32_t *dptrs, const int32
     if (B <= 0) throw_error(SILI_ERR_INVALID, "backward_sparse: batch must be >= 1");
     if (!x || !dptrs || !dx) throw_error(SILI_ERR_INVALID, "backward_sparse: NULL buffer");
     launch_colabs(x, B, L.n_in, L.acc_in.p, st);
-    L.ws_gT.ensure((size_t)(L.n_out * B));
+    L.ws_gT.ensure((size_t)(L.n_out * B + BATCH_SLACK));
     launch_densify_full(dptrs, didx, dvals, B, L.n_out, L.ws_gT.p, L.acc_grad.p, true, nnz_dy, st);
     launch_zero_split_rows(L.W.plan(), dx, L.n_in, B, st);
     // scattered: merge-join visits only present dy entries (sisldo_ops.hpp:705-713);
@@ -769,7 +769,7 @@ void backward_sparse_train(Layer &L, const float *x, const int32_t *dptrs, const
     const float *xT = to_feature_major(L, L.ws_xT, x, B, L.n_in, nullptr, st);
     L.xT_cached_batch = 0;
     launch_rowabs(xT, B, L.n_in, L.acc_in.p, st);
-    L.ws_gT.ensure((size_t)(L.n_out * B));
+    L.ws_gT.ensure((size_t)(L.n_out * B + BATCH_SLACK));
     // entries present in dy carry nonzero bits (explicit zeros as -0.0)
     launch_densify_full(dptrs, didx, dvals, B, L.n_out, L.ws_gT.p, L.acc_grad.p, true, nnz_dy, st);
     ensure_train_state(L, st);

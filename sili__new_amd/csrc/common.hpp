@@ -214,6 +214,10 @@ struct Block4Plan {
     bool has_split;
 };
 
+// Floats that a feature-major copy [n][B] is longer than n * B: the float4
+// kernels read a row of a batch that is no multiple of 4 past its end.
+constexpr int64_t BATCH_SLACK = 4;
+
 // out[b*out_ld + row] for b < nb: scattered gather (stores; atomics for split
 // rows -- then the caller has zeroed out).  in is feature-major in[c*in_ld + b].
 // accumulate: add to out (batches with nb % 4 == 0 and aligned feature-major

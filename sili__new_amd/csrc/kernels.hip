@@ -19,6 +19,7 @@
 #include "wave.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <cstdlib>
 
 namespace sili {
@@ -530,12 +531,18 @@ __device__ __forceinline__ uint32_t decode_segment_entries(const StagedSeg &sg, 
     return n;
 }
 
-// float4 along the batch: groups of BL lanes take one entry each (G = 64/BL
+// float4 along the batch, for every batch from 2 on (a lane per batch column, as
+// k_gather has it, is 64 columns wide at any batch and loads 4 bytes a lane:
+// forward, grad-input and grad-W at 3001 x 5003, 2 %, batch 37 46.7 us with it
+// and k_sddmm, 25.0 with these kernels; batch 3 21.1 / 16.6, 127 83.4 / 38.6).
+// Groups of BL lanes take one entry each (G = 64/BL
 // entries per load instruction); lane bl of a group owns float4 chunks
 // q = bl + BL*k (k < KB) of the entry's feature-major input row.  The whole
 // segment is decoded first (decode_segment_entries); the gather loop then
-// keeps U loads per lane in flight with no predicates.  Needs nb % 4 == 0,
-// in_ld % 4 == 0 and a 16-byte aligned `in`.
+// keeps U loads per lane in flight with no predicates.  A batch that is no
+// multiple of 4 reads into the next row with its last chunk (rows are 4-byte
+// aligned then, as buffer loads allow, and the input has BATCH_SLACK floats
+// more): those columns are not stored.
 constexpr uint32_t ENT_CAP = SEG_BYTES_MAX + 64u;
 
 // Block epilogue of the float4 kernels: out[b, row] for the block's (up to
@@ -570,7 +577,7 @@ constexpr int WAITCNT_VM0 = 0x0F70;
 
 template <int BL, int KB>
 __device__ __forceinline__ void store_rows_block(const float4 (&acc)[KB], bool active, uint32_t row,
-                                                 bool split, uint32_t nq, float *slice_base,
+                                                 bool split, uint32_t nb, float *slice_base,
                                                  uint32_t slice_stride, float *out, int64_t out_ld,
                                                  bool accumulate = false,
                                                  SplitCombine sc = SplitCombine{nullptr, 0, nullptr, nullptr, nullptr},
@@ -585,7 +592,7 @@ __device__ __forceinline__ void store_rows_block(const float4 (&acc)[KB], bool a
 #pragma unroll
         for (int k = 0; k < KB; ++k) {
             const uint32_t q = bl + BL * (uint32_t)k;
-            if (q < nq) *reinterpret_cast<float4 *>(slice + q * 4u) = acc[k];
+            if (q * 4u < nb) *reinterpret_cast<float4 *>(slice + q * 4u) = acc[k];
         }
     }
     if (lane == 0) {
@@ -593,7 +600,6 @@ __device__ __forceinline__ void store_rows_block(const float4 (&acc)[KB], bool a
         s_flag[wave] = (active ? 1u : 0u) | (split && !combine ? 2u : 0u) | (combine ? 4u : 0u);
     }
     __syncthreads();
-    const uint32_t nb = nq * 4u;
     for (uint32_t i = threadIdx.x; i < nb * WAVES; i += blockDim.x) {
         const uint32_t w = i % WAVES, b = i / WAVES;
         const uint32_t f = s_flag[w];
@@ -665,7 +671,7 @@ __device__ __forceinline__ void gather_short_body(const GArgs &a, uint32_t sblk,
     constexpr uint32_t US = KB * RPG >= 4u ? 1u : 2u;     // entries per row in flight
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.nb >> 2), nbv = nq * 4u;
+    const uint32_t nq = (uint32_t)(a.nb + 3) >> 2, nbv = nq * 4u;
     const int64_t i0 = ((int64_t)sblk * WAVES + wave) * SHORT_R_MAX;
     const uint32_t nrows = i0 < a.n_sh ? (uint32_t)min<int64_t>((int64_t)SHORT_R_MAX, a.n_sh - i0) : 0u;
     SegStage &S = stage[wave];
@@ -817,7 +823,7 @@ __device__ __forceinline__ void gather_short_body(const GArgs &a, uint32_t sblk,
     __syncthreads();
     // the block's rows per batch index: consecutive threads on consecutive rows
     constexpr uint32_t PER_B = WAVES * SHORT_R_MAX;
-    for (uint32_t i = threadIdx.x; i < nbv * PER_B; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < (uint32_t)a.nb * PER_B; i += blockDim.x) {
         const uint32_t r = i % SHORT_R_MAX, w = (i / SHORT_R_MAX) % WAVES, b = i / PER_B;
         if (r >= stage[w].idx[SHORT_R_MAX]) continue;
         const float v = reinterpret_cast<const float *>(ents[w])[r * nbv + b];
@@ -846,7 +852,7 @@ void k_gather_v4(GArgs a) {
     const int64_t si = (int64_t)bid * WAVES + wave;
     const bool active = si < a.nseg;  // inactive waves still join the block epilogue
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.nb >> 2);
+    const uint32_t nq = (uint32_t)(a.nb + 3) >> 2;
     float4 acc[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -905,7 +911,7 @@ void k_gather_v4(GArgs a) {
         }
     wave_lds_sync();  // the entry table is reused as this wave's output slice
     }
-    store_rows_block<BL, KB>(acc, active, sd.row, (sd.split & SEG_SPLIT) != 0, nq,
+    store_rows_block<BL, KB>(acc, active, sd.row, (sd.split & SEG_SPLIT) != 0, (uint32_t)a.nb,
                              reinterpret_cast<float *>(&s_ent[0][0]), ENT_CAP * 2u, a.out, a.out_ld,
                              a.accumulate != 0, SplitCombine{a.seg, a.nseg, a.elem_start, a.split_cnt, a.part},
                              si, sd.elem_end - sd.elem_begin);
@@ -1215,14 +1221,20 @@ struct FArgs {
     float *part;
 };
 
+// The first n (0 or more than 4: all) of v's floats, the others 0.
+__device__ __forceinline__ float4 first_of(float4 v, uint32_t n) {
+    return make_float4(v.x, n == 1u ? 0.0f : v.y, n - 1u < 2u ? 0.0f : v.z, n - 1u < 3u ? 0.0f : v.w);
+}
+
 // Fused grad-input + nnz-sampled grad-W over the canonical store: one decode
 // of the segment, one load of gT[col] per entry, used twice --
 //   dx[b,row] += w_e * gT[col_e,b]        (the grad-input gather)
 //   gw[e]      = sum_b xT[row,b]*gT[col_e,b] (the sampled grad-W)
 // Lane layout as k_gather_v4 (BL lanes per entry, float4 chunks of the
-// batch), xT[row] in registers as k_sddmm_v4.  Needs B % 4 == 0, 16-byte
-// aligned xT / gT and B <= 64*KB*4/ (64/BL) -- the launcher checks.
-template <int BL, int KB, int U>
+// batch), xT[row] in registers as k_sddmm_v4.  TAIL: B % 4 != 0, the last
+// chunk's columns past the batch set to 0; else xT / gT are 16-byte aligned.
+// Needs B <= 64*KB*4/ (64/BL) -- the launcher checks.
+template <int BL, int KB, int U, bool TAIL>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, 256), amdgpu_waves_per_eu(KB <= 2 && KB * U <= 4 ? 8 : 1)))
 void k_bwd_v4(FArgs a) {
     __shared__ SegStage s_stage[WAVES];
@@ -1235,7 +1247,7 @@ void k_bwd_v4(FArgs a) {
     const int64_t si = (int64_t)bid * WAVES + wave;
     const bool active = si < a.nseg;  // inactive waves still join the block epilogue
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.B >> 2);
+    const uint32_t nq = (uint32_t)(a.B + 3) >> 2;
     float4 acc[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1245,7 +1257,7 @@ void k_bwd_v4(FArgs a) {
     fp4_table_init(s_fp4[wave]);
     const StagedSeg sg = stage_segment(s_stage[wave], a.idx, a.val, sd);
     const __amdgpu_buffer_rsrc_t rg = buffer_rsrc(a.gT, a.gT_bytes);
-    const float4 *x4p = reinterpret_cast<const float4 *>(a.xT) + (int64_t)sd.row * nq;
+    const float *xrow = a.xT + (int64_t)sd.row * a.B;
     uint32_t lane_off[KB];
     float4 xr[KB];
     float part = 0.0f;
@@ -1253,7 +1265,8 @@ void k_bwd_v4(FArgs a) {
     for (int k = 0; k < KB; ++k) {
         const uint32_t q = bl + BL * (uint32_t)k;
         lane_off[k] = q < nq ? q * 16u : OOB_OFFSET;
-        xr[k] = q < nq ? x4p[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (TAIL) xr[k] = q < nq ? first_of(load_f4(xrow + q * 4u), (uint32_t)a.B - q * 4u) : make_float4(0.f, 0.f, 0.f, 0.f);
+        else xr[k] = q < nq ? reinterpret_cast<const float4 *>(xrow)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
         part += (__builtin_fabsf(xr[k].x) + __builtin_fabsf(xr[k].y)) +
                 (__builtin_fabsf(xr[k].z) + __builtin_fabsf(xr[k].w));
     }
@@ -1272,6 +1285,14 @@ void k_bwd_v4(FArgs a) {
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int k = 0; k < KB; ++k) gv[u][k] = buffer_load_f4(rg, e[u].x + lane_off[k]);
+        if constexpr (TAIL) {
+            // the next row's values must not meet the products below, where
+            // even a zero does not stop an infinity
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int k = 0; k < KB; ++k) gv[u][k] = first_of(gv[u][k], (uint32_t)a.B - (bl + BL * (uint32_t)k) * 4u);
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float w = __builtin_bit_cast(float, e[u].y);
@@ -1303,7 +1324,7 @@ void k_bwd_v4(FArgs a) {
         }
     wave_lds_sync();  // the entry table is reused as this wave's output slice
     }
-    store_rows_block<BL, KB>(acc, active, sd.row, (sd.split & SEG_SPLIT) != 0, nq,
+    store_rows_block<BL, KB>(acc, active, sd.row, (sd.split & SEG_SPLIT) != 0, (uint32_t)a.B,
                              reinterpret_cast<float *>(&s_ent[0][0]), ENT_CAP * 2u, a.dx, a.dx_ld, false,
                              SplitCombine{a.seg, a.nseg, a.elem_start, a.split_cnt, a.part}, si,
                              sd.elem_end - sd.elem_begin);
@@ -1345,8 +1366,8 @@ __device__ __forceinline__ void store_rows4_block(bool active, uint32_t brow, bo
 // decodes a tile dequantises its 16 slots into LDS (one 16-byte tile load);
 // then G = 64/BL tiles per load instruction, U tiles per group in flight,
 // each lane loading the 4 input rows 4bc+lj of its tile (float4 chunks of
-// the batch) and accumulating the tile's 4 output rows.  Needs nb % 4 == 0,
-// in_ld % 4 == 0, a 16-byte aligned `in` and a < 2 GiB input.
+// the batch) and accumulating the tile's 4 output rows (nb % 4 != 0: as in
+// k_gather_v4; the slack is finite).  Needs a < 2 GiB input.
 template <int BL, int KB, int U>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(U <= 2 ? 4 : 1))) void k_gather_b4_v4(BArgs a, uint32_t in_bytes) {
     __shared__ uint32_t s_off[WAVES][64];
@@ -1366,7 +1387,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(U <= 2 ? 4 
     const int64_t si = (int64_t)bx * WAVES + wave;
     const bool active = si < a.nseg;
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.nb >> 2);
+    const uint32_t nq = (uint32_t)(a.nb + 3) >> 2;
     const uint32_t q0 = by * (BL * KB);
     float4 acc[4][KB];
 #pragma unroll
@@ -1547,7 +1568,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     const int64_t si = (int64_t)blockIdx.x * WAVES + wave;
     const bool active = si < a.nseg;
     const uint32_t lj = lane >> 4, bl = lane & 15u;
-    const uint32_t nq = (uint32_t)(a.nb >> 2);
+    const uint32_t nq = (uint32_t)(a.nb + 3) >> 2;
     const uint32_t q0 = blockIdx.y * 16u;
     float4 acc[4];
 #pragma unroll
@@ -1851,9 +1872,9 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_mfma(SBArgs a, uint32_t gT_byt
 // batch (B = 4*BL*KB at most): xT's 4 rows of the block row stay in
 // registers; G = 64/BL tiles per load instruction, each lane loading the 4
 // gT rows of its tile and forming 16 partial dots, reduced over the BL
-// batch lanes; the group's last lane stores the tile's 64 bytes.  Needs
-// B % 4 == 0, 16-byte aligned xT / gT / gw and a < 2 GiB gT.
-template <int BL, int KB>
+// batch lanes; the group's last lane stores the tile's 64 bytes.  TAIL: as in
+// k_bwd_v4.  Needs 16-byte aligned gw and a < 2 GiB gT.
+template <int BL, int KB, bool TAIL>
 __global__ __launch_bounds__(256) void k_sddmm_b4_v4(SBArgs a, uint32_t gT_bytes) {
     __shared__ uint32_t s_off[WAVES][64];
     __shared__ uint32_t s_t[WAVES][64];
@@ -1863,7 +1884,7 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_v4(SBArgs a, uint32_t gT_bytes
     if (si >= a.nseg) return;
     const SegDesc sd = a.seg[si];
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.B >> 2);
+    const uint32_t nq = (uint32_t)(a.B + 3) >> 2;
     const uint32_t ld_bytes = (uint32_t)a.B * 4u;
     const __amdgpu_buffer_rsrc_t rg = buffer_rsrc(a.gT, gT_bytes);
     uint32_t lane_off[KB];
@@ -1875,8 +1896,11 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_v4(SBArgs a, uint32_t gT_bytes
 #pragma unroll
         for (int li = 0; li < 4; ++li) {
             const int64_t r = (int64_t)sd.row * 4 + li;
-            xr[li][k] = (q < nq && r < a.rows)
-                ? reinterpret_cast<const float4 *>(a.xT + r * a.B)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+            xr[li][k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (q < nq && r < a.rows) {
+                if constexpr (TAIL) xr[li][k] = first_of(load_f4(a.xT + r * a.B + q * 4u), (uint32_t)a.B - q * 4u);
+                else xr[li][k] = reinterpret_cast<const float4 *>(a.xT + r * a.B)[q];
+            }
         }
     }
     uint32_t pos = sd.byte_begin, carry = sd.base_col, ebase = sd.elem_begin;
@@ -1898,7 +1922,10 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_v4(SBArgs a, uint32_t gT_bytes
             for (int lj = 0; lj < 4; ++lj) {
                 float4 gv[KB];
 #pragma unroll
-                for (int k = 0; k < KB; ++k) gv[k] = buffer_load_f4(rg, off + (uint32_t)lj * ld_bytes + lane_off[k]);
+                for (int k = 0; k < KB; ++k) {
+                    gv[k] = buffer_load_f4(rg, off + (uint32_t)lj * ld_bytes + lane_off[k]);
+                    if constexpr (TAIL) gv[k] = first_of(gv[k], (uint32_t)a.B - (bl + BL * (uint32_t)k) * 4u);
+                }
 #pragma unroll
                 for (int li = 0; li < 4; ++li) {
                     // one chain per slot (16 independent chains per lane)
@@ -1915,6 +1942,11 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_v4(SBArgs a, uint32_t gT_bytes
             }
 #pragma unroll
             for (int s = 0; s < 16; ++s) d[s] = group_sum_last<BL>(d[s]);
+            if constexpr (TAIL) {  // an edge tile's slots outside the layer: 0
+#pragma unroll
+                for (int s = 0; s < 16; ++s)
+                    if ((int64_t)sd.row * 4 + s % 4 >= a.rows || off + (uint32_t)(s / 4) * ld_bytes >= gT_bytes - BATCH_SLACK * 4) d[s] = 0.0f;
+            }
             if (bl == BL - 1u && e < n) {
                 float4 *o = reinterpret_cast<float4 *>(a.gw + (size_t)s_t[wave][e] * 16u);
                 o[0] = make_float4(d[0], d[1], d[2], d[3]);
@@ -1943,7 +1975,7 @@ struct SRArgs {
     int64_t B;
     float *gw;
 };
-template <int BL, int KB>
+template <int BL, int KB, bool TAIL>
 __global__ __launch_bounds__(256) void k_sddmm_b4_rng(SRArgs a, uint32_t gT_bytes) {
     constexpr uint32_t G = 64u / BL;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
@@ -1953,7 +1985,7 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_rng(SRArgs a, uint32_t gT_byte
     const uint32_t t0 = a.start[run], t1 = a.start[run + a.brows];
     if (t0 >= t1) return;
     const uint32_t g = lane / BL, bl = lane % BL;
-    const uint32_t nq = (uint32_t)(a.B >> 2);
+    const uint32_t nq = (uint32_t)(a.B + 3) >> 2;
     const uint32_t ld_bytes = (uint32_t)a.B * 4u;
     const __amdgpu_buffer_rsrc_t rg = buffer_rsrc(a.gT, gT_bytes);
     uint32_t lane_off[KB];
@@ -1965,8 +1997,11 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_rng(SRArgs a, uint32_t gT_byte
 #pragma unroll
         for (int li = 0; li < 4; ++li) {
             const int64_t r = br * 4 + li;
-            xr[li][k] = (q < nq && r < a.rows)
-                ? reinterpret_cast<const float4 *>(a.xT + r * a.B)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+            xr[li][k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (q < nq && r < a.rows) {
+                if constexpr (TAIL) xr[li][k] = first_of(load_f4(a.xT + r * a.B + q * 4u), (uint32_t)a.B - q * 4u);
+                else xr[li][k] = reinterpret_cast<const float4 *>(a.xT + r * a.B)[q];
+            }
         }
     }
     for (uint32_t j = t0; j < t1; j += G) {
@@ -1978,7 +2013,10 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_rng(SRArgs a, uint32_t gT_byte
         for (int lj = 0; lj < 4; ++lj) {
             float4 gv[KB];
 #pragma unroll
-            for (int k = 0; k < KB; ++k) gv[k] = buffer_load_f4(rg, off + (uint32_t)lj * ld_bytes + lane_off[k]);
+            for (int k = 0; k < KB; ++k) {
+                gv[k] = buffer_load_f4(rg, off + (uint32_t)lj * ld_bytes + lane_off[k]);
+                if constexpr (TAIL) gv[k] = first_of(gv[k], (uint32_t)a.B - (bl + BL * (uint32_t)k) * 4u);
+            }
 #pragma unroll
             for (int li = 0; li < 4; ++li) {
                 // one chain per slot (16 independent chains per lane)
@@ -1995,6 +2033,11 @@ __global__ __launch_bounds__(256) void k_sddmm_b4_rng(SRArgs a, uint32_t gT_byte
         }
 #pragma unroll
         for (int s = 0; s < 16; ++s) d[s] = group_sum_last<BL>(d[s]);
+        if constexpr (TAIL) {  // an edge tile's slots outside the layer: 0
+#pragma unroll
+            for (int s = 0; s < 16; ++s)
+                if (br * 4 + s % 4 >= a.rows || off + (uint32_t)(s / 4) * ld_bytes >= gT_bytes - BATCH_SLACK * 4) d[s] = 0.0f;
+        }
         if (bl == BL - 1u && ok) {
             float4 *o = reinterpret_cast<float4 *>(a.gw + (size_t)t * 16u);
             o[0] = make_float4(d[0], d[1], d[2], d[3]);
@@ -2093,6 +2136,8 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ src
             if (j < n && b < B) dst[j * B + b] = tile[bb][jj + 4u * i];
         }
     }
+    // (an edge tile of the block4 gather multiplies them by 0)
+    if (B % 4 != 0 && blockIdx.x == 0 && blockIdx.y == 0 && t < (uint32_t)BATCH_SLACK) dst[n * B + t] = 0.0f;
 }
 
 // The same with float4 rows: a 64(b) x 32(j) tile, 128-byte reads along j,
@@ -2515,13 +2560,12 @@ void launch_gather(const GatherPlan &p, const ScaleView &sc, const float *in, in
     ProfScope ps("gather", st);
     for (int64_t b0 = 0; b0 < nb_total; b0 += 512) {
         const int64_t nb = nb_total - b0 < 512 ? nb_total - b0 : 512;
-        const int64_t in_bytes = (p.cols * in_ld - b0) * 4;
+        const int64_t in_bytes = (p.cols * in_ld - b0) * 4 + (in_ld % 4 ? BATCH_SLACK * 4 : 0);
         const bool small = in_bytes < (int64_t)OOB_OFFSET;
+        const bool v4 = small && nb > 1;
         GArgs a{p.seg, p.nseg, p.idx, p.val, sc, in + b0, in_ld, out + b0 * out_ld, out_ld, nb,
                 small ? (uint32_t)in_bytes : 0u, accumulate ? 1 : 0, xcd_order(0), nullptr, nullptr, nullptr};
-        if (accumulate && !(small && nb % 4 == 0 && in_ld % 4 == 0 && aligned16(a.in)))
-            throw_error(3, "launch_gather: accumulating passes need the float4 kernels");
-        const bool v4 = small && nb % 4 == 0 && in_ld % 4 == 0 && aligned16(a.in);
+        if (accumulate && !v4) throw_error(3, "launch_gather: accumulating passes need the float4 kernels");
         if (v4 && p.has_split && p.part && p.nseg * nb <= p.part_cap) {
             a.elem_start = p.elem_start;
             a.split_cnt = p.split_cnt;
@@ -2587,7 +2631,7 @@ void launch_gather(const GatherPlan &p, const ScaleView &sc, const float *in, in
                 }
             }
         } else if (v4) {
-            const int64_t nq = nb / 4;
+            const int64_t nq = (nb + 3) / 4;
             if (nq <= 1) gather_v4_skip<1, 1>(a, skip, st);
             else if (nq <= 2) gather_v4_skip<2, 1>(a, skip, st);
             else if (nq <= 4) gather_v4_skip<4, 1>(a, skip, st);
@@ -2623,11 +2667,10 @@ void launch_gather_b4(const Block4Plan &p, const ScaleView &sc, const float *in,
                       float *out, int64_t out_ld, int64_t nb_total, int skip, hipStream_t st) {
     if (p.nseg == 0 || nb_total == 0) return;
     ProfScope ps("gather_b4", st);
-    const int64_t in_bytes = p.cols * in_ld * 4;
-    if (skip == SKIP_NONE && nb_total % 4 == 0 && in_ld % 4 == 0 && aligned16(in) &&
-        in_bytes < (int64_t)OOB_OFFSET) {
+    const int64_t in_bytes = p.cols * in_ld * 4 + (in_ld % 4 ? BATCH_SLACK * 4 : 0);
+    if (skip == SKIP_NONE && nb_total > 1 && in_bytes < (int64_t)OOB_OFFSET) {
         BArgs a{p.seg, p.nseg, p.idx, p.tiles, p.rows, p.cols, sc, in, in_ld, out, out_ld, nb_total};
-        const int64_t nq = nb_total / 4;
+        const int64_t nq = (nb_total + 3) / 4;
         const unsigned gx = blocks_for(p.nseg);
         const unsigned gy16 = (unsigned)((nq + 15) / 16);
         const int use_mfma = env_int("SILI_B4_MFMA", 0);  // (knobs read per call)
@@ -2733,8 +2776,9 @@ void launch_sddmm(const GatherPlan &p, const float *xT, const float *gT, int64_t
 
 bool launch_bwd_fused(const GatherPlan &p, const ScaleView &sc, const float *gT, const float *xT,
                       int64_t B, float *dx, int64_t dx_ld, float *gw, float *acc_in, hipStream_t st) {
-    const int64_t gT_bytes = p.cols * B * 4;
-    if (B % 4 != 0 || B > 512 || gT_bytes >= (int64_t)OOB_OFFSET || !aligned16(xT) || !aligned16(gT))
+    const int64_t gT_bytes = p.cols * B * 4 + (B % 4 ? BATCH_SLACK * 4 : 0);
+    const bool tail = B % 4 != 0;
+    if (B < 2 || B > 512 || gT_bytes >= (int64_t)OOB_OFFSET || (!tail && (!aligned16(xT) || !aligned16(gT))))
         return false;
     if (p.nseg == 0) return true;
     ProfScope ps("gather_gradw", st);
@@ -2746,31 +2790,36 @@ bool launch_bwd_fused(const GatherPlan &p, const ScaleView &sc, const float *gT,
         a.part = p.part;
     }
     const dim3 grid(blocks_for(p.nseg)), block(256);
-    const int64_t nq = B / 4;
-    if (nq <= 1) launch((k_bwd_v4<1, 1, 4>), grid, block, 0, st, a);
-    else if (nq <= 2) launch((k_bwd_v4<2, 1, 4>), grid, block, 0, st, a);
-    else if (nq <= 4) launch((k_bwd_v4<4, 1, 4>), grid, block, 0, st, a);
-    else if (nq <= 8) launch((k_bwd_v4<8, 1, 4>), grid, block, 0, st, a);
-    else if (nq <= 16) {
-        const int bl = gather_bl(), u = gather_u();
-        if (nq > 8 && bl == 4) {
-            if (u >= 2) launch((k_bwd_v4<4, 4, 2>), grid, block, 0, st, a);
-            else launch((k_bwd_v4<4, 4, 1>), grid, block, 0, st, a);
-        } else if (nq > 8 && bl == 8) {
-            // 2 entries per group in flight: 60 VGPRs, so 8 waves per SIMD
-            // (4 in flight: 80 VGPRs, 6 waves; 22.6 against 26.1 us on the
-            // config-1 grad-input + grad-W)
-            if (u >= 4) launch((k_bwd_v4<8, 2, 4>), grid, block, 0, st, a);
-            else launch((k_bwd_v4<8, 2, 2>), grid, block, 0, st, a);
-        } else launch((k_bwd_v4<16, 1, 4>), grid, block, 0, st, a);
-    } else if (nq <= 32) {
-        const int bl = gather_bl();
-        if (bl == 4) launch((k_bwd_v4<4, 8, 1>), grid, block, 0, st, a);
-        else if (bl == 8) launch((k_bwd_v4<8, 4, 1>), grid, block, 0, st, a);
-        else launch((k_bwd_v4<16, 2, 4>), grid, block, 0, st, a);
-    }
-    else if (nq <= 64) launch((k_bwd_v4<16, 4, 2>), grid, block, 0, st, a);
-    else launch((k_bwd_v4<16, 8, 1>), grid, block, 0, st, a);
+    const int64_t nq = (B + 3) / 4;
+    auto go = [&](auto odd) {
+        constexpr bool T = decltype(odd)::value;
+        if (nq <= 1) launch((k_bwd_v4<1, 1, 4, T>), grid, block, 0, st, a);
+        else if (nq <= 2) launch((k_bwd_v4<2, 1, 4, T>), grid, block, 0, st, a);
+        else if (nq <= 4) launch((k_bwd_v4<4, 1, 4, T>), grid, block, 0, st, a);
+        else if (nq <= 8) launch((k_bwd_v4<8, 1, 4, T>), grid, block, 0, st, a);
+        else if (nq <= 16) {
+            const int bl = gather_bl(), u = gather_u();
+            if (nq > 8 && bl == 4) {
+                if (u >= 2) launch((k_bwd_v4<4, 4, 2, T>), grid, block, 0, st, a);
+                else launch((k_bwd_v4<4, 4, 1, T>), grid, block, 0, st, a);
+            } else if (nq > 8 && bl == 8) {
+                // 2 entries per group in flight: 60 VGPRs, so 8 waves per SIMD
+                // (4 in flight: 80 VGPRs, 6 waves; 22.6 against 26.1 us on the
+                // config-1 grad-input + grad-W)
+                if (u >= 4) launch((k_bwd_v4<8, 2, 4, T>), grid, block, 0, st, a);
+                else launch((k_bwd_v4<8, 2, 2, T>), grid, block, 0, st, a);
+            } else launch((k_bwd_v4<16, 1, 4, T>), grid, block, 0, st, a);
+        } else if (nq <= 32) {
+            const int bl = gather_bl();
+            if (bl == 4) launch((k_bwd_v4<4, 8, 1, T>), grid, block, 0, st, a);
+            else if (bl == 8) launch((k_bwd_v4<8, 4, 1, T>), grid, block, 0, st, a);
+            else launch((k_bwd_v4<16, 2, 4, T>), grid, block, 0, st, a);
+        }
+        else if (nq <= 64) launch((k_bwd_v4<16, 4, 2, T>), grid, block, 0, st, a);
+        else launch((k_bwd_v4<16, 8, 1, T>), grid, block, 0, st, a);
+    };
+    if (tail) go(std::true_type{});
+    else go(std::false_type{});
     SILI_HIP(hipGetLastError());
     return true;
 }
@@ -2780,33 +2829,46 @@ void launch_sddmm_b4(const Block4Plan &p, const B4Ranges *rng, const float *xT, 
     if (p.nseg == 0) return;
     ProfScope ps("sddmm_b4", st);
     SBArgs a{p.seg, p.nseg, p.idx, p.rows, p.cols, xT, gT, B, gw};
-    const int64_t gT_bytes = p.cols * B * 4;
-    if (B % 4 == 0 && B <= 256 && gT_bytes < (int64_t)OOB_OFFSET && aligned16(xT) && aligned16(gT) &&
-        aligned16(gw)) {
+    const bool tail = B % 4 != 0;
+    const int64_t gT_bytes = p.cols * B * 4 + (tail ? BATCH_SLACK * 4 : 0);
+    if (B > 1 && B <= 256 && gT_bytes < (int64_t)OOB_OFFSET && aligned16(gw) &&
+        (tail || (aligned16(xT) && aligned16(gT)))) {
         const dim3 grid(blocks_for(p.nseg)), block(256);
-        const int64_t nq = B / 4;
+        const int64_t nq = (B + 3) / 4;
         if (rng && rng->K >= 1 && rng->tcol && rng->start) {
             const int64_t nruns = rng->K * rng->brows;
             SRArgs r{rng->tcol, rng->start, nruns, rng->brows, p.rows, xT, gT, B, gw};
             const dim3 rgrid(blocks_for(nruns));
-            if (nq <= 4) launch((k_sddmm_b4_rng<4, 1>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
-            else if (nq <= 8) launch((k_sddmm_b4_rng<8, 1>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
-            else if (nq <= 16) launch((k_sddmm_b4_rng<16, 1>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
-            else if (nq <= 32) launch((k_sddmm_b4_rng<16, 2>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
-            else launch((k_sddmm_b4_rng<16, 4>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+            auto go = [&](auto odd) {
+                constexpr bool T = decltype(odd)::value;
+                if (nq <= 4) launch((k_sddmm_b4_rng<4, 1, T>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+                else if (nq <= 8) launch((k_sddmm_b4_rng<8, 1, T>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+                else if (nq <= 16) launch((k_sddmm_b4_rng<16, 1, T>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+                else if (nq <= 32) launch((k_sddmm_b4_rng<16, 2, T>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+                else launch((k_sddmm_b4_rng<16, 4, T>), rgrid, block, 0, st, r, (uint32_t)gT_bytes);
+            };
+            if (tail) go(std::true_type{});
+            else go(std::false_type{});
             SILI_HIP(hipGetLastError());
             return;
         }
         const int use_mfma = env_int("SILI_B4_MFMA", 0);  // (knobs read per call)
-        if (use_mfma && nq >= 8) {
+        if (use_mfma && nq >= 8 && !tail) {
             if (nq <= 16) launch((k_sddmm_b4_mfma<1, 2>), grid, block, 0, st, a, (uint32_t)gT_bytes);
             else if (nq <= 32) launch((k_sddmm_b4_mfma<2, 2>), grid, block, 0, st, a, (uint32_t)gT_bytes);
             else launch((k_sddmm_b4_mfma<4, 2>), grid, block, 0, st, a, (uint32_t)gT_bytes);
-        } else if (nq <= 4) launch((k_sddmm_b4_v4<4, 1>), grid, block, 0, st, a, (uint32_t)gT_bytes);
-        else if (nq <= 8) launch((k_sddmm_b4_v4<8, 1>), grid, block, 0, st, a, (uint32_t)gT_bytes);
-        else if (nq <= 16) launch((k_sddmm_b4_v4<16, 1>), grid, block, 0, st, a, (uint32_t)gT_bytes);
-        else if (nq <= 32) launch((k_sddmm_b4_v4<16, 2>), grid, block, 0, st, a, (uint32_t)gT_bytes);
-        else launch((k_sddmm_b4_v4<16, 4>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+        } else {
+            auto go = [&](auto odd) {
+                constexpr bool T = decltype(odd)::value;
+                if (nq <= 4) launch((k_sddmm_b4_v4<4, 1, T>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+                else if (nq <= 8) launch((k_sddmm_b4_v4<8, 1, T>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+                else if (nq <= 16) launch((k_sddmm_b4_v4<16, 1, T>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+                else if (nq <= 32) launch((k_sddmm_b4_v4<16, 2, T>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+                else launch((k_sddmm_b4_v4<16, 4, T>), grid, block, 0, st, a, (uint32_t)gT_bytes);
+            };
+            if (tail) go(std::true_type{});
+            else go(std::false_type{});
+        }
         SILI_HIP(hipGetLastError());
         return;
     }

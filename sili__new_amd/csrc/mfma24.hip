@@ -243,6 +243,8 @@ __global__ __launch_bounds__(256) void k_m24_split(SplitArgs a) {
         }
     }
     if (!ok) *a.flag = a.epoch;
+    // (as in k_transpose)
+    if (a.xT && a.B % 4 != 0 && blockIdx.x == 0 && threadIdx.x < (uint32_t)BATCH_SLACK) a.xT[a.cols * a.B + threadIdx.x] = 0.0f;
     uint4 *o = reinterpret_cast<uint4 *>(a.out);
     struct Two {
         uint4 lo, hi;
