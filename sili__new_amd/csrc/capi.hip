@@ -492,8 +492,8 @@ void forward_dense(Layer &L, const float *x, int64_t B, float *y, hipStream_t st
     // backward_dense reads when called without x (sili/cpu_backend.cpp:481)
     L.xT_cached_batch = B > 1 ? B : 0;
     const bool str = L.Wt.nnz > 0 && !m24 && stream_wanted(L.Wt, ssc, B, B, skip);
-    // batches 65..128: the input staged in LDS slice by slice (SILI_STAGED)
-    const bool staged = L.Wt.nnz > 0 && !m24 && !str && env_int("SILI_STAGED", 1) && staged_supported(L, L.Wt, ssc, xT, B, skip);
+    // batches 65..128: the input staged in LDS slice by slice
+    const bool staged = L.Wt.nnz > 0 && !m24 && !str && staged_supported(L, L.Wt, ssc, xT, B, skip) && staged_wanted(L.Wt, B);
     const bool plain = L.Wt.nnz > 0 && !m24 && !str && !staged && colblock_passes(L.Wt, xT, B) == 0;
     if (L.Wt.nnz == 0) prep.fill(y, B * L.n_out, 0.0f);
     else if (plain) prep.zero_split(L.Wt.plan(), y, L.n_out, B);

@@ -676,6 +676,13 @@ void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb);
 // The staged-input gather (staged.hip): whether it takes this case, and
 // out[b, r] for every row r of s (written, not added).
 bool staged_supported(const Layer &L, const DScatter &s, const ScaleView &sc, const float *in, int64_t B, int skip);
+// Estimated times in us of the staged gather and of the segment gather (with its
+// column-block passes) at batch B, and whether the first is taken where it can.
+double staged_us(const DScatter &s);
+inline double segments_us(const DScatter &s, int64_t B) {
+    return 8.0 + (double)s.nnz * std::max(5.3e-6, 2.2e-6 + 1.45e-7 * (double)B);
+}
+bool staged_wanted(const DScatter &s, int64_t B);
 void launch_gather_staged(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t B, float *out,
                           int64_t out_ld, hipStream_t st);
 // The matrix-core gather (mfma24.hip): whether it takes this case (its copy of

@@ -829,7 +829,8 @@ double others_us(const DScatter &s, int64_t B) {
         const double blocks = std::ceil((double)(s.cols + 1) * (double)B * 4.0 / 150e3);
         return 6.0 + 1.5 * (double)B * blocks + 0.14e-6 * (double)B * nnz;
     }
-    return 8.0 + nnz * std::max(5.3e-6, 2.2e-6 + 1.45e-7 * (double)B);
+    if (B > 64 && B <= 128 && B % 4 == 0 && staged_wanted(s, B)) return std::min(segments_us(s, B), staged_us(s));
+    return segments_us(s, B);
 }
 
 }  // namespace

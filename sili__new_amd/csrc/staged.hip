@@ -22,6 +22,7 @@
 #include "wave.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace sili {
 
@@ -241,6 +242,29 @@ bool staged_supported(const Layer &L, const DScatter &s, const ScaleView &sc, co
     return s.nnz > 0 && s.nnz < (int64_t(1) << 32) && B > 64 && B <= (int64_t)SL_B && B % 4 == 0 &&
            sc.rank == 1 && skip == SKIP_NONE && (reinterpret_cast<uintptr_t>(in) & 15u) == 0 &&
            s.rows * (S + 1) <= s.nnz;
+}
+
+// Its time in us: SL_R rows a block, one block a CU; a slice costs a block 4.3 us
+// (the copy, the barriers) and 51 us times the density (128 x 256 cells).
+double staged_us(const DScatter &s) {
+    const double d = (double)s.nnz / ((double)s.rows * (double)s.cols);
+    const double rounds = std::ceil((double)s.rows / ((double)SL_R * 256.0));
+    return 10.0 + rounds * std::ceil((double)s.cols / (double)SL_W) * (4.3 + 51.0 * d);
+}
+
+// A block waits for its whole slice however few synapses read from it, so the
+// segment gather is ahead on layers of few blocks or low density.  us, staged /
+// segments, batch 128: 700 x 1000 at 3 % 36 / 8, 4096^2 at 2 % 95 / 19, at 6 % 126
+// / 30, 8192^2 at 2 % 167 / 40, at 10 % 297 / 160, 16384^2 at 2 % 316 / 167, 4096 x
+// 32768 at 2 % 97 / 64, at 4 % 113 / 107; the other way round 4096 x 65536 at 10 %
+// 315 / 468, 5120 x 204800 at 10 % 1335 / 2185 (estimated).  The estimates are
+// fitted below 10 %; from 25 % on the older rule (staging wherever it can run)
+// stands, although it is behind on layers of few rows there too (16384 x 300 at
+// 40 % 1632 / 140).
+bool staged_wanted(const DScatter &s, int64_t B) {
+    const int mode = env_int("SILI_STAGED", 2);  // (read per call) 0 never, 1 whenever it can, 2 by the above
+    if (mode != 2) return mode != 0;
+    return (double)s.nnz >= 0.25 * (double)s.rows * (double)s.cols || staged_us(s) < segments_us(s, B);
 }
 
 void ensure_slices(Layer &L, DScatter &s, hipStream_t st) {

@@ -100,3 +100,18 @@ def test_wide_sparse_layer_stays_on_segment_gather(hip):
     counts = kernel_counts(hip, L, lambda: assert_close_terms(
         L.forward_dense(x), H.forward_dense(x), H.forward_dense(x, absmode=True), "wide sparse B128"))
     assert "fwd:gather_staged" not in counts and "fwd:slices" not in counts, counts
+
+
+@pytest.mark.parametrize("n_in,n_out,density,staged", [(2048, 2048, 0.03, False), (300, 60000, 0.2, True),
+                                                       (4096, 64, 0.3, True)])
+def test_staged_where_it_is_ahead(hip, monkeypatch, n_in, n_out, density, staged):
+    """The default takes the segment gather where a slice holds little work for
+    its block, and staging on layers of many rows or from 25 % density on; both
+    match the oracle."""
+    from tests.test_gpu_stream import kernel_counts
+    monkeypatch.delenv("SILI_STAGED", raising=False)
+    H, L = make(hip, n_in, n_out, density, 9)
+    x = np.random.default_rng(10).normal(size=(128, n_in)).astype(np.float32)
+    counts = kernel_counts(hip, L, lambda: assert_close_terms(
+        L.forward_dense(x), H.forward_dense(x), H.forward_dense(x, absmode=True), f"{n_in}x{n_out}"))
+    assert ("fwd:gather_staged" in counts) == staged, counts
