@@ -939,10 +939,11 @@ __global__ void k_cb_flag(const uint32_t *__restrict__ cols, int64_t N, uint32_t
 __global__ void k_cb_take(const uint32_t *__restrict__ flag, const uint32_t *__restrict__ pos,
                           const uint32_t *__restrict__ rows, const uint32_t *__restrict__ cols,
                           const uint8_t *__restrict__ val, int64_t N, uint32_t c0, uint32_t *__restrict__ rk,
-                          uint32_t *__restrict__ ck, uint8_t *__restrict__ vk) {
+                          uint32_t *__restrict__ ck, uint8_t *__restrict__ vk, uint32_t *__restrict__ src) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= N || !flag[i]) return;
     const uint32_t j = pos[i];
+    if (src) src[j] = (uint32_t)i;
     rk[j] = rows[i];
     ck[j] = cols[i] - c0;
     vk[j] = val[i];
@@ -951,8 +952,9 @@ __global__ void k_cb_take(const uint32_t *__restrict__ flag, const uint32_t *__r
 void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb) {
     hipStream_t st = L.stream;
     const int64_t N = s.nnz;
-    DevBuf<uint32_t> rows, cols, flag, pos, rk, ck, ptrs;
+    DevBuf<uint32_t> rows, cols, flag, pos, rk, ck, ptrs, src;
     DevBuf<uint8_t> vk;
+    if (L.keep_perm) src.ensure((size_t)N + 1);  // a layer that trains refreshes the copies' values
     rows.ensure((size_t)N + 1);
     cols.ensure((size_t)N + 1);
     flag.ensure((size_t)N + 1);
@@ -976,14 +978,40 @@ void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb) {
         if (N > 0)
             launch(k_cb_take, dim3(nblk(N)), dim3(TPB), 0, st, (const uint32_t *)flag.p, (const uint32_t *)pos.p,
                    (const uint32_t *)rows.p, (const uint32_t *)cols.p, (const uint8_t *)s.val.p, N, (uint32_t)c0,
-                   rk.p, ck.p, vk.p);
+                   rk.p, ck.p, vk.p, src.p);
         launch(k_ptrs_from_sorted, dim3(nblk(s.rows + 1)), dim3(TPB), 0, st, (const uint32_t *)rk.p, (int64_t)nk,
                s.rows, ptrs.p);
         SILI_HIP(hipGetLastError());
         build_scattered(L, blocks[(size_t)k], s.rows, ncols, (int64_t)nk, ptrs.p, ck.p, vk.p);
+        if (src.p) {
+            blocks[(size_t)k].from.ensure((size_t)nk + 1);
+            SILI_HIP(hipMemcpyAsync(blocks[(size_t)k].from.p, src.p, (size_t)nk * 4, hipMemcpyDeviceToDevice, st));
+        }
     }
+    SILI_HIP(hipStreamSynchronize(st));  // src is freed on return
     s.cblk = std::move(blocks);
     s.cblk_cb = cb;
+    s.cblk_stale = false;
+}
+
+void refresh_colblocks(DScatter &s, hipStream_t st) {
+    ProfScope ps("colblock_values", st);
+    for (DScatter &b : s.cblk)
+        if (b.nnz > 0)
+            launch(k_gather_u8, dim3(nblk(b.nnz)), dim3(TPB), 0, st, (const uint8_t *)s.val.p, (const uint32_t *)b.from.p,
+                   b.nnz, b.val.p);
+    SILI_HIP(hipGetLastError());
+    s.cblk_stale = false;
+}
+
+void refresh_colblocks_b4(DBlock4 &s, hipStream_t st) {
+    ProfScope ps("colblock_values", st);
+    for (DBlock4 &b : s.cblk)
+        if (b.ntiles > 0)
+            launch(k_gather_tiles, dim3(nblk(b.ntiles)), dim3(TPB), 0, st, (const uint8_t *)s.tiles.p,
+                   (const uint32_t *)b.from.p, b.ntiles, 0, b.tiles.p);
+    SILI_HIP(hipGetLastError());
+    s.cblk_stale = false;
 }
 
 // One orientation of block4 from tiles sorted by (major, minor).
@@ -1062,10 +1090,13 @@ void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb) {
         SILI_HIP(hipGetLastError());
         build_b4_orientation(L, blocks[(size_t)k], (int64_t)nt, b.brows, nbc, b.rows, ncols, mk.p, nk.p, pk.p,
                              b.tiles.p, false);
+        blocks[(size_t)k].from.ensure((size_t)nt + 1);
+        SILI_HIP(hipMemcpyAsync(blocks[(size_t)k].from.p, pk.p, (size_t)nt * 4, hipMemcpyDeviceToDevice, st));
     }
     SILI_HIP(hipStreamSynchronize(st));
     b.cblk = std::move(blocks);
     b.cblk_cbb = cbb;
+    b.cblk_stale = false;
 }
 
 // start[x*brows + br] = the first tile of block row br whose block column

@@ -436,6 +436,7 @@ bool gather_colblocked(Layer &L, DScatter &s, const ScaleView &sc, const float *
     if (K == 0) return false;
     const int64_t cb = (s.cols + K - 1) / K;
     if ((int64_t)s.cblk.size() != K || s.cblk_cb != cb) build_colblocks(L, s, (int)K, cb);
+    else if (s.cblk_stale) refresh_colblocks(s, st);
     for (int64_t k = 0; k < K; ++k) {
         DScatter &sub = s.cblk[(size_t)k];
         const int64_t c0 = k * cb;
@@ -464,6 +465,7 @@ bool gather_b4_colblocked(Layer &L, DBlock4 &b, const ScaleView &sc, const float
     if (K < 2) return false;
     const int64_t cbb = (b.bcols + K - 1) / K;
     if ((int64_t)b.cblk.size() != K || b.cblk_cbb != cbb) build_colblocks_b4(L, b, (int)K, cbb);
+    else if (b.cblk_stale) refresh_colblocks_b4(b, st);
     for (int64_t k = 0; k < K; ++k) {
         const int64_t c0 = k * cbb * 4;
         const ScaleView sk{sc.row, sc.ent ? sc.ent + c0 * sc.rank : nullptr, sc.rank};
@@ -680,7 +682,9 @@ void backward_dense_train(Layer &L, const float *x, const float *dy, int64_t B, 
     ensure_shadow_perm(L);
     if (L.output_scale_trainable) L.mterm.ensure((size_t)(L.W.nnz * 2 * L.rank));
     const uint64_t seed = splitmix64_host(L.rng_seed ^ splitmix64_host(L.rng_calls + 1));
-    launch_train_rows(L, xT, gT, B, dx, p, seed, st);
+    // (a wave per row writing its zeros: 24.6 us at 16384 rows, batch 256)
+    if (L.W.nnz == 0) fill(dx, B * L.n_in, 0.0f, st);
+    else launch_train_rows(L, xT, gT, B, dx, p, seed, st);
     // block4 tiles after the scattered rows' scale steps (linear_disldo.hpp:962-1951)
     launch_train_b4(L, xT, gT, B, dx, p, seed, st);
     // the update rewrites every tile: each is re-encoded by its live count
@@ -694,16 +698,15 @@ void backward_dense_train(Layer &L, const float *x, const float *dy, int64_t B, 
     launch_train_store(L, seed, st);
     launch_shadow_val_refresh(L, st);
     launch_b4_shadow_refresh(L, st);
-    // copies holding value bytes are stale now: rebuilt on their next use
+    // copies holding value bytes are stale now: rebuilt, or their values
+    // gathered again, on their next use
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
         sc->drop_m24();
-        sc->cblk.clear();
-        sc->cblk_cb = 0;
+        sc->values_changed();
     }
     for (DBlock4 *b4 : {&L.B4, &L.B4t}) {
-        b4->cblk.clear();
-        b4->cblk_cbb = 0;
+        b4->cblk_stale = true;
     }
     L.vs_ones = false;
     if (L.output_scale_trainable && scales_step) L.os_ones = false;
@@ -789,12 +792,10 @@ void backward_sparse_train(Layer &L, const float *x, const int32_t *dptrs, const
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
         sc->drop_m24();
-        sc->cblk.clear();
-        sc->cblk_cb = 0;
+        sc->values_changed();
     }
     for (DBlock4 *b4 : {&L.B4, &L.B4t}) {
-        b4->cblk.clear();
-        b4->cblk_cbb = 0;
+        b4->cblk_stale = true;
     }
     L.vs_ones = false;
     ++L.train_calls;

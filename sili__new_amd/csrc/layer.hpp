@@ -140,6 +140,18 @@ struct DScatter {
     // columns relative to the block (built on first use)
     std::vector<DScatter> cblk;
     int64_t cblk_cb = 0;
+    // an update changes values, not places: a copy keeps its entries' places in
+    // the store (from) and takes the new values on its next use (cblk_stale),
+    // where building it anew costs a decode, K scans and K encodings
+    DevBuf<uint32_t> from;
+    bool cblk_stale = false;
+    void values_changed() {
+        cblk_stale = true;
+        if (!cblk.empty() && !cblk[0].from.p) {
+            cblk.clear();
+            cblk_cb = 0;
+        }
+    }
     // split rows combined in item order by the float4 gather: arrivals per
     // row (rows+1, zero between launches) and per-item partial sums
     // (part_cap floats; empty: combined by atomics)
@@ -183,6 +195,8 @@ struct DBlock4 {
     // column-block copies (as DScatter::cblk, in block columns of cblk_cbb)
     std::vector<DBlock4> cblk;
     int64_t cblk_cbb = 0;
+    DevBuf<uint32_t> from;  // (as DScatter::from: tiles)
+    bool cblk_stale = false;
     // the tiles by column range (built on first use, kept until the structure
     // changes): each tile's block column, and for range x of rng_k and block
     // row br the first tile of the row in that range, rng_start[x*brows + br]
@@ -671,6 +685,8 @@ void device_sort_pairs_u64(Layer &L, const uint64_t *kin, uint64_t *kout, const 
 
 // Column-block copies of s (s.cblk, K blocks of cb columns; block4: cbb
 // block columns).
+void refresh_colblocks(DScatter &s, hipStream_t st);
+void refresh_colblocks_b4(DBlock4 &s, hipStream_t st);
 void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb);
 void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb);
 // The staged-input gather (staged.hip): whether it takes this case, and

@@ -100,3 +100,45 @@ def test_block4_column_blocks(hip, monkeypatch, n_in, n_out, op):
         assert_close_terms(dx, H.backward_dense(x, g)[0], H.backward_dense(x, g, absmode=True)[0], "b4 colblock dx")
     counts = kernel_counts(hip, L, run)
     assert counts.get(f"{op}:gather_b4") == 4, counts
+
+
+def test_column_blocks_follow_updates(hip, monkeypatch):
+    """The copies' values are gathered again after an optimizer step (scattered
+    and block4), not built anew, and a structural change drops them: the same
+    outputs as without passes, step by step."""
+    from tests.test_gpu_parity import _edge_block4_layer
+    br, bc, tiles, ptrs, cols, q, vs = _edge_block4_layer(16387, 70, 17, density=0.03)
+    layers = []
+    for _ in range(2):
+        L = hip.SparseLinearLayer(16387, 70, 8 * len(cols) + 64 * len(br) + 4096)
+        L.load_weights(ptrs, cols, q)
+        L.load_block4_tiles(br, bc, tiles)
+        L.set_value_scales(vs)
+        layers.append(L)
+    rng = np.random.default_rng(3)
+    seen = []
+    for step in range(5):
+        x = rng.normal(size=(136, 16387)).astype(np.float32)
+        g = rng.normal(size=(136, 70)).astype(np.float32)
+        got = []
+        for mode, L in zip("10", layers):
+            monkeypatch.setenv("SILI_COLBLOCK", mode)
+            out = {}
+            counts = kernel_counts(hip, L, lambda: out.update(y=L.forward_dense(x)))
+            if mode == "1":
+                seen.append(counts.get("fwd:colblock_values", 0))
+            out["dx"] = L.backward_dense(g, 0.05)
+            got.append(out)
+            if step == 3:
+                cr = np.arange(0, 16000, 16, dtype=np.int32)
+                L.synapto_step(0.1, cr, cr % 70, np.full(len(cr), 0.3, np.float32))
+        a, b = (L.export_scattered()["val"] for L in layers)
+        assert np.array_equal(a, b), step
+        for k in ("y", "dx"):
+            # the fp32 bar, 1e-5 of the summed magnitudes, which are at least the largest output; a
+            # stale value is off by a code's step times its scale and input, over 0.1
+            np.testing.assert_allclose(got[0][k], got[1][k], rtol=0, atol=1e-5 * np.abs(got[0][k]).max(),
+                                       err_msg=f"{k} step {step}")
+    # a launch per copy, 5 scattered and 2 block4: built at first, the scattered ones once more after the first
+    # update, which makes the layer keep places; then the values; built anew after the structure changed
+    assert seen == [0, 2, 7, 7, 0], seen
