@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <array>
+#include <bitset>
 #include <cstring>
 #include <map>
 #include <string>
@@ -130,10 +131,15 @@ struct DScatter {
     // us it saved or would have saved since the values last changed, and when
     // to build it: m24_saved >= m24_cost * m24_wait
     double m24_saved = 0, m24_cost = 0, m24_wait = 1;
+    // batches that the other kernels have served since then: what they build on
+    // first use is there, so a call under stream capture, which takes them,
+    // builds nothing
+    std::bitset<513> m24_warm;
     void drop_m24() {
         if (m24_valid) m24_wait = m24_saved < m24_cost * (m24_wait + 1) ? std::min(m24_wait * 2, 1e6) : 1;
         m24_valid = false;
         m24_saved = 0;
+        m24_warm.reset();
     }
     // column-block copies for gathers whose operand exceeds one XCD's L2:
     // cblk[k] holds every row's entries with columns in [k*cblk_cb, ...),

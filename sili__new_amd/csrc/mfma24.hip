@@ -905,6 +905,8 @@ static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
 // copy was dropped before it had paid for itself: a layer used a few times or
 // trained between its forwards keeps the other paths.  Under stream capture
 // never: a graph would go on reading the copy after the weights have changed.
+// The first call of each batch takes the other kernels, which leaves a program
+// that runs a batch before it captures it all that the captured call needs.
 bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int skip, hipStream_t st) {
     // SILI_MFMA24 (read per call): 0 never, 2 whenever it can and at once, 1
     // (default) by the estimates
@@ -919,10 +921,10 @@ bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int sk
         const double g = gain();
         if (Shape(s).cells * 0.375 > 8e9 || g < 0) return false;
         s.m24_saved += g + 0.1 * other;
-        if (!s.m24_valid) {
-            s.m24_cost = 500.0 + 1.7e-5 * (double)s.nnz;
-            if (s.m24_saved < s.m24_cost * s.m24_wait) return false;
-        }
+        if (!s.m24_valid) s.m24_cost = 500.0 + 1.7e-5 * (double)s.nnz;
+        const bool warm = s.m24_warm.test((size_t)B);
+        s.m24_warm.set((size_t)B);
+        if (!warm || (!s.m24_valid && s.m24_saved < s.m24_cost * s.m24_wait)) return false;
     }
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     SILI_HIP(hipStreamIsCapturing(st, &cap));

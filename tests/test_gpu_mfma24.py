@@ -5,10 +5,13 @@ turn), empty rows, groups of 4 columns with 3 and 4 entries (the overflow list)
 up to full rows, batches around the operand tiles (10 and 21 for the pieces as
 columns, 32, 64, 128 a chunk), inputs without an exact split (non-finite, tiny),
 and the copy's life: built late, dropped when values or structure change."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle import HostLayer
+from tests.test_gpu_capi import Api, _ptr
 from tests.test_gpu_stream import kernel_counts
 from tests.util import assert_close_terms
 
@@ -143,3 +146,53 @@ def test_mfma24_is_built_when_it_pays(hip, monkeypatch):
     small = make(hip, 300, 400, 0.2, 5, False)[1]
     xs = rng.normal(size=(64, 300)).astype(np.float32)
     assert all("fwd:mfma24" not in kernel_counts(hip, small, lambda: small.forward_dense(xs)) for _ in range(20))
+
+
+def test_mfma24_leaves_what_a_captured_call_needs(hip, monkeypatch):
+    """A batch that ran twice before it is captured: the captured call takes the
+    other kernels, whose first use builds and waits, so the first of those runs
+    took them too, although another batch had the copy built by then.  The graph
+    is replayed on new inputs between eager calls."""
+    monkeypatch.delenv("SILI_MFMA24", raising=False)
+    api = Api(hip.LIB_PATH)
+    H, L = make(hip, 1000, 8192, 0.3, 6, False, full=False)
+    rng = np.random.default_rng(8)
+    xw = rng.normal(size=(128, 1000)).astype(np.float32)
+    for _ in range(60):
+        L.forward_dense(xw)
+    assert kernel_counts(hip, L, lambda: L.forward_dense(xw)).get("fwd:mfma24", 0) == 1
+    B, h = 64, C.c_void_p(L.handle)
+    x, y, st, graph, run = (C.c_void_p() for _ in range(5))
+    rt = lambda name, *args: api.ck(getattr(api.L, name)(*args))  # the HIP runtime that the library is linked to
+    rt("sili_device_alloc", h, B * 1000 * 4, C.byref(x))
+    rt("sili_device_alloc", h, B * 8192 * 4, C.byref(y))
+    rt("hipStreamCreate", C.byref(st))
+    got = np.empty((B, 8192), np.float32)
+
+    def forward():
+        rt("sili_forward_dense", h, x, B, y, st)
+
+    def result(call):
+        v = rng.normal(size=(B, 1000)).astype(np.float32)
+        got[:] = np.nan
+        rt("sili_memcpy_h2d", h, x, _ptr(v), v.nbytes)
+        rt("sili_memcpy_h2d", h, y, _ptr(got), got.nbytes)
+        call()
+        rt("hipStreamSynchronize", st)
+        rt("sili_memcpy_d2h", h, _ptr(got), y, got.nbytes)
+        assert_close_terms(got, H.forward_dense(v), H.forward_dense(v, absmode=True), "replay")
+
+    assert "fwd:mfma24" not in kernel_counts(hip, L, lambda: result(forward))
+    assert kernel_counts(hip, L, lambda: result(forward)).get("fwd:mfma24", 0) == 1
+    rt("hipStreamBeginCapture", st, 0)
+    forward()
+    rt("hipStreamEndCapture", st, C.byref(graph))
+    rt("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+    for _ in range(3):
+        result(lambda: rt("hipGraphLaunch", run, st))
+        result(forward)
+    rt("hipGraphExecDestroy", run)
+    rt("hipGraphDestroy", graph)
+    rt("hipStreamDestroy", st)
+    rt("sili_device_free", h, x)
+    rt("sili_device_free", h, y)
