@@ -695,7 +695,7 @@ struct B4TrainArgs {
     uint64_t seed;
 };
 
-// One block of 4 waves per canonical block row (linear_disldo.hpp:962-1951,
+// One block of W = 4 waves per canonical block row (linear_disldo.hpp:962-1951,
 // FP4): every slot of the row's tiles trains.  A lane holds one tile row
 // (lane = 4 * tile + li; a wave takes 16 tiles at a time, the block 64): its
 // 4 slots are 4 independent chains of batch steps, and the sums over a tile
@@ -709,8 +709,10 @@ struct B4TrainArgs {
 // the tile rows' sums turn in LDS and 16 lanes add them in tile order, as the
 // reference does (an LDS float add with several lanes per address took 150
 // clocks a wave); the waves' rows are added in wave order at the end.
-constexpr uint32_t WAVES_B4 = 4;  // waves per block of k_train_b4
-constexpr uint32_t TILES_B4 = 16 * WAVES_B4;  // tiles the block takes at a time
+//
+// W = 1, a block of one wave: for rows of 16 tiles or fewer on average, whose
+// other waves would have nothing to step and keep blocks off the chip
+// (the rule stands at launch_b4_rank).
 // Floats of a row of batch values in LDS: 16-byte aligned, and 4 more so that
 // the 4 rows' reads of one step group fall into different banks.
 constexpr uint32_t TURN_LD = 20;  // a (row, step)'s 16 tiles in LDS, 16-byte aligned
@@ -724,11 +726,12 @@ struct B4State {
     float mc[COLS ? 4 : 1][2 * RANK];
 };
 
-template <int RANK, bool COLS>
-__global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4TrainArgs a) {
-    __shared__ double s_mr[TILES_B4][4][2 * RANK];  // [tile][li][k | contrib k]
+template <int RANK, bool COLS, uint32_t W>
+__global__ __launch_bounds__(64 * W, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4TrainArgs a) {
+    constexpr uint32_t TILES = 16 * W;  // tiles the block takes at a time
+    __shared__ double s_mr[TILES][4][2 * RANK];  // [tile][li][k | contrib k]
     __shared__ double s_row[4][2 * RANK];           // the rows' sums over all tiles
-    __shared__ __attribute__((aligned(16))) float s_turn[WAVES_B4][16 * TURN_LD];
+    __shared__ __attribute__((aligned(16))) float s_turn[W][16 * TURN_LD];
     extern __shared__ __attribute__((aligned(16))) float s_dyn[];  // x [4][LD], then dx [wave][4][LD]
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const int64_t br = blockIdx.x;
@@ -736,7 +739,7 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
     if (t0 == t1) return;  // the whole block
     const int64_t B = a.B, LD = b4_ld(B);
     float *sx = s_dyn, *sdx = s_dyn + (1 + wave) * 4 * LD, *sturn = s_turn[wave];
-    for (int64_t i = threadIdx.x; i < 4 * LD; i += 256) {
+    for (int64_t i = threadIdx.x; i < 4 * LD; i += 64 * W) {
         const int64_t l = i / LD, b = i % LD;
         sx[i] = b < B && br * 4 + l < a.n_in ? a.xT[(br * 4 + l) * B + b] : 0.0f;
     }
@@ -754,7 +757,7 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
     for (int k = 0; k < RANK; ++k) vs_k[k] = row_ok ? a.vs[row * RANK + k] : 0.0f;
     const float imp_scale = (a.is && row_ok) ? a.is[row] : 1.0f;
     const float *xl = sx + li * LD;
-    for (uint32_t p0 = t0; p0 < t1; p0 += TILES_B4) {
+    for (uint32_t p0 = t0; p0 < t1; p0 += TILES) {
         const uint32_t tw = p0 + wave * 16u;  // the wave's first tile
         if (tw < t1) {
             const bool tile_ok = tw + tl < t1;
@@ -882,13 +885,19 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
                 }
                 wave_lds_sync();
             };
-            int64_t b = 0;
+            // a group's 4 batch values of slot j; the last group's load reads on
+            // into the next row (gT has BATCH_SLACK floats more, except at batch 1)
+            auto load4 = [&](int j, int64_t b) {
+                return B > 1 ? load_f4(g0 + j * B + b) : make_float4(g0[j], 0.0f, 0.0f, 0.0f);
+            };
             float4 nx[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                nx[j] = fast && B >= 4 ? load_f4(g0 + j * B) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            for (; b + 4 <= B; b += 4) {
-                float dx4[4];
+            for (int j = 0; j < 4; ++j) nx[j] = fast ? load4(j, 0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            // 4 batch steps at a time, the last 1..3 as a shorter group (LDS rows
+            // hold b4_ld(B) > B + 3 floats)
+            auto group = [&](auto whole, int64_t b) {
+                const int n = decltype(whole)::value ? 4 : (int)(B - b);
+                float dx4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                 bool done = false;
                 if (fast) {
                     const B4State<RANK, COLS> keep = s;
@@ -901,12 +910,12 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
                         dy[1][j] = nx[j].y;
                         dy[2][j] = nx[j].z;
                         dy[3][j] = nx[j].w;
-                        if (b + 8 <= B) nx[j] = load_f4(g0 + j * B + b + 4);
+                        if (b + 4 < B) nx[j] = load4(j, b + 4);
                     }
                     StepRange rg;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        dx4[i] = fast_step(x[i], dy[i], rg);
+                        if (i < n) dx4[i] = fast_step(x[i], dy[i], rg);
                         // the 4 slots' chains interleave; interleaving steps too
                         // only costs registers (spills at 4 waves per SIMD)
                         __builtin_amdgcn_sched_barrier(0);
@@ -916,7 +925,7 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
                 }
                 if (!done) {
 #pragma unroll 1
-                    for (int i = 0; i < 4; ++i) {
+                    for (int i = 0; i < n; ++i) {
                         const float d = exact_step(b + i);
                         dx4[0] = i == 0 ? d : dx4[0];
                         dx4[1] = i == 1 ? d : dx4[1];
@@ -927,20 +936,10 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
 #pragma unroll
                 for (int i = 0; i < 4; ++i) dx4[i] = lane_on ? dx4[i] : 0.0f;
                 add_dx(b, dx4);
-            }
-            if (b < B) {  // the last 1..3 steps (LDS rows hold b4_ld(B) > B + 3 floats)
-                float dx4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-                for (int64_t i = 0; b + i < B; ++i) {
-                    const float d = exact_step(b + i);
-                    dx4[0] = i == 0 ? d : dx4[0];
-                    dx4[1] = i == 1 ? d : dx4[1];
-                    dx4[2] = i == 2 ? d : dx4[2];
-                }
-#pragma unroll
-                for (int i = 0; i < 3; ++i) dx4[i] = lane_on ? dx4[i] : 0.0f;
-                add_dx(b, dx4);
-            }
+            };
+            int64_t b = 0;
+            for (; b + 4 <= B; b += 4) group(std::true_type{}, b);
+            if (b < B) group(std::false_type{}, b);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if (!has[j]) continue;
@@ -968,19 +967,19 @@ __global__ __launch_bounds__(256, RANK == 1 && !COLS ? 4 : 2) void k_train_b4(B4
         // the tile rows' fp64 partials, added per row in tile order
         if (threadIdx.x < 8u * RANK) {
             const uint32_t l = threadIdx.x / (2u * RANK), k = threadIdx.x % (2u * RANK);
-            const uint32_t n = min(TILES_B4, t1 - p0);
+            const uint32_t n = min(TILES, t1 - p0);
             double sum = s_row[l][k];
             for (uint32_t u = 0; u < n; ++u) sum = sum + s_mr[u][l][k];
             s_row[l][k] = sum;
         }
         __syncthreads();
     }
-    for (int64_t i = threadIdx.x; i < 4 * B; i += 256) {
+    for (int64_t i = threadIdx.x; i < 4 * B; i += 64 * W) {
         const int64_t l = i & 3, b = i >> 2, rr = br * 4 + l;
         if (rr >= a.n_in) continue;
         float v = 0.0f;
 #pragma unroll
-        for (uint32_t w = 0; w < WAVES_B4; ++w) v += s_dyn[((1 + w) * 4 + l) * LD + b];
+        for (uint32_t w = 0; w < W; ++w) v += s_dyn[((1 + w) * 4 + l) * LD + b];
         a.dx[b * a.n_in + rr] += v;
     }
     // the block rows' scale step (linear_disldo.hpp:1923-1951)
@@ -1464,17 +1463,21 @@ void launch_rows_kernel(int rank, bool deferred, bool cols, dim3 grid, dim3 bloc
     }
 }
 
+// One wave a block while a row has at most a wave's 16 tiles on average, else 4.
+// Training step, 9216 x 2816 with 8.5 tiles a row, us: with 4 waves / with 1:
+// batch 1 57.7 / 46.9, 2 57.9 / 47.0, 5 63.6 / 51.9, 13 77.0 / 63.8.
 template <int RANK>
-void launch_b4_rank(const B4TrainArgs &a, hipStream_t st) {
+void launch_b4_rank(const B4TrainArgs &a, int64_t ntiles, hipStream_t st) {
+    const uint32_t waves = ntiles <= 16 * a.brows ? 1u : 4u;
     // x and each wave's dx rows: up to 82 KB at batch 1024
-    const uint32_t lds = (uint32_t)((1 + WAVES_B4) * 4 * b4_ld(a.B) * sizeof(float));
+    const uint32_t lds = (uint32_t)((1 + waves) * 4 * b4_ld(a.B) * sizeof(float));
     auto go = [&](auto kernel) {
         SILI_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds));
-        launch(kernel, dim3((unsigned)a.brows), dim3(64 * WAVES_B4), lds, st, a);
+        launch(kernel, dim3((unsigned)a.brows), dim3(64 * waves), lds, st, a);
     };
-    if (a.b4term) go(&k_train_b4<RANK, true>);
-    else go(&k_train_b4<RANK, false>);
+    if (waves == 1u) a.b4term ? go(&k_train_b4<RANK, true, 1>) : go(&k_train_b4<RANK, false, 1>);
+    else a.b4term ? go(&k_train_b4<RANK, true, 4>) : go(&k_train_b4<RANK, false, 4>);
 }
 
 }  // namespace
@@ -1661,10 +1664,10 @@ void launch_train_b4(Layer &L, const float *xT, const float *gT, int64_t B, floa
     a.seed = seed;
     ProfScope ps("train_b4", st);
     switch (L.rank) {
-        case 1: launch_b4_rank<1>(a, st); break;
-        case 2: launch_b4_rank<2>(a, st); break;
-        case 3: launch_b4_rank<3>(a, st); break;
-        default: launch_b4_rank<4>(a, st); break;
+        case 1: launch_b4_rank<1>(a, L.B4.ntiles, st); break;
+        case 2: launch_b4_rank<2>(a, L.B4.ntiles, st); break;
+        case 3: launch_b4_rank<3>(a, L.B4.ntiles, st); break;
+        default: launch_b4_rank<4>(a, L.B4.ntiles, st); break;
     }
     SILI_HIP(hipGetLastError());
 }
