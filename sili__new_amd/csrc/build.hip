@@ -839,7 +839,6 @@ void build_scattered(Layer &L, DScatter &dst, int64_t rows, int64_t ncols, int64
     dst.m24_failed = false;
     dst.stream1.failed = dst.streamK.failed = false;
     dst.cblk.clear();
-    dst.cblk_cb = 0;
     dst.rows = rows;
     dst.cols = ncols;
     dst.nnz = N;
@@ -903,7 +902,6 @@ void build_shadow(Layer &L, const DScatter &src, const uint32_t *d_rows, const u
     dst.drop_m24();
     dst.m24_failed = false;
     dst.cblk.clear();
-    dst.cblk_cb = 0;
     dst.rows = src.cols;
     dst.cols = src.rows;
     dst.nnz = N;
@@ -949,7 +947,7 @@ __global__ void k_cb_take(const uint32_t *__restrict__ flag, const uint32_t *__r
     vk[j] = val[i];
 }
 
-void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb) {
+static ColBlocks<DScatter> build_colblocks(Layer &L, DScatter &s, int64_t K, int64_t cb) {
     hipStream_t st = L.stream;
     const int64_t N = s.nnz;
     DevBuf<uint32_t> rows, cols, flag, pos, rk, ck, ptrs, src;
@@ -989,29 +987,25 @@ void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb) {
         }
     }
     SILI_HIP(hipStreamSynchronize(st));  // src is freed on return
-    s.cblk = std::move(blocks);
-    s.cblk_cb = cb;
-    s.cblk_stale = false;
+    return ColBlocks<DScatter>{std::move(blocks), cb};
 }
 
-void refresh_colblocks(DScatter &s, hipStream_t st) {
+static void refresh_colblocks(DScatter &s, ColBlocks<DScatter> &c, hipStream_t st) {
     ProfScope ps("colblock_values", st);
-    for (DScatter &b : s.cblk)
+    for (DScatter &b : c.block)
         if (b.nnz > 0)
             launch(k_gather_u8, dim3(nblk(b.nnz)), dim3(TPB), 0, st, (const uint8_t *)s.val.p, (const uint32_t *)b.from.p,
                    b.nnz, b.val.p);
     SILI_HIP(hipGetLastError());
-    s.cblk_stale = false;
 }
 
-void refresh_colblocks_b4(DBlock4 &s, hipStream_t st) {
+static void refresh_colblocks(DBlock4 &s, ColBlocks<DBlock4> &c, hipStream_t st) {
     ProfScope ps("colblock_values", st);
-    for (DBlock4 &b : s.cblk)
+    for (DBlock4 &b : c.block)
         if (b.ntiles > 0)
             launch(k_gather_tiles, dim3(nblk(b.ntiles)), dim3(TPB), 0, st, (const uint8_t *)s.tiles.p,
                    (const uint32_t *)b.from.p, b.ntiles, 0, b.tiles.p);
     SILI_HIP(hipGetLastError());
-    s.cblk_stale = false;
 }
 
 // One orientation of block4 from tiles sorted by (major, minor).
@@ -1037,7 +1031,6 @@ static void build_b4_orientation(Layer &L, DBlock4 &dst, int64_t N, int64_t brow
     dst.has_split = e.has_split;
     dst.tiles.ensure((size_t)N * 16u + 64);
     dst.cblk.clear();
-    dst.cblk_cbb = 0;
     dst.rng_k = 0;
     if (N > 0) {
         launch(k_gather_tiles, dim3(nblk(N)), dim3(TPB), 0, st, d_src_tiles, d_perm, N,
@@ -1060,7 +1053,7 @@ __global__ void k_cb4_take(const uint32_t *__restrict__ flag, const uint32_t *__
     pk[j] = (uint32_t)i;
 }
 
-void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb) {
+static ColBlocks<DBlock4> build_colblocks(Layer &L, DBlock4 &b, int64_t K, int64_t cbb) {
     hipStream_t st = L.stream;
     const int64_t N = b.ntiles;
     DevBuf<uint32_t> major, minor, flag, pos, mk, nk, pk;
@@ -1094,9 +1087,58 @@ void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb) {
         SILI_HIP(hipMemcpyAsync(blocks[(size_t)k].from.p, pk.p, (size_t)nt * 4, hipMemcpyDeviceToDevice, st));
     }
     SILI_HIP(hipStreamSynchronize(st));
-    b.cblk = std::move(blocks);
-    b.cblk_cbb = cbb;
-    b.cblk_stale = false;
+    return ColBlocks<DBlock4>{std::move(blocks), cbb};
+}
+
+template <typename Store>
+static const ColBlocks<Store> *find_colblocks(Layer &L, Store &s, int64_t K, int64_t width, hipStream_t st) {
+    const bool cap = capturing(st);
+    for (ColBlocks<Store> &c : s.cblk) {
+        if ((int64_t)c.block.size() != K || c.width != width) continue;
+        if (c.stale) {
+            // (recorded, a refresh would not have run when the next call
+            // gathers from these copies)
+            if (cap) return nullptr;
+            refresh_colblocks(s, c, st);
+            c.stale = false;
+        }
+        c.captured |= cap;
+        return &c;
+    }
+    if (cap) return nullptr;
+    s.cblk.erase(std::remove_if(s.cblk.begin(), s.cblk.end(), [](const ColBlocks<Store> &c) { return !c.captured; }),
+                 s.cblk.end());
+    s.cblk.push_back(build_colblocks(L, s, K, width));
+    return &s.cblk.back();
+}
+const ColBlocks<DScatter> *colblocks(Layer &L, DScatter &s, int64_t K, int64_t width, hipStream_t st) {
+    return find_colblocks(L, s, K, width, st);
+}
+const ColBlocks<DBlock4> *colblocks(Layer &L, DBlock4 &s, int64_t K, int64_t width, hipStream_t st) {
+    return find_colblocks(L, s, K, width, st);
+}
+
+template <typename Store>
+static void changed(Store &s, bool cap, hipStream_t st) {
+    // copies built before the layer trained know no places
+    s.cblk.erase(std::remove_if(s.cblk.begin(), s.cblk.end(),
+                                [](const ColBlocks<Store> &c) { return !c.block[0].from.p; }),
+                 s.cblk.end());
+    for (ColBlocks<Store> &c : s.cblk) {
+        c.stale = true;
+        if (c.captured && !cap) {
+            refresh_colblocks(s, c, st);
+            c.stale = false;
+        }
+    }
+}
+void colblock_values_changed(Layer &L, hipStream_t st) {
+    if (L.W.cblk.empty() && L.Wt.cblk.empty() && L.B4.cblk.empty() && L.B4t.cblk.empty()) return;
+    const bool cap = capturing(st);
+    changed(L.W, cap, st);
+    changed(L.Wt, cap, st);
+    changed(L.B4, cap, st);
+    changed(L.B4t, cap, st);
 }
 
 // start[x*brows + br] = the first tile of block row br whose block column

@@ -415,37 +415,30 @@ struct Prep {
 
 }  // namespace
 
-// Column-block passes of a scattered gather over s, or 0 when they do not
-// apply.  SILI_COLBLOCK (read per call): 0 never, else when the gathered
+// SILI_COLBLOCK (read per call): 0 no column-block passes, else when the gathered
 // operand is larger than 4 MiB (one XCD's L2); passes of <= SILI_COLBLOCK_MB
 // (default 2 MiB: measured on c4's down layer at batch 128, 8 passes of
 // 2 MiB beat 4 of 4 MiB and 2 of 8 MiB).
-int64_t colblock_passes(const DScatter &s, const float *in, int64_t B) {
+const ColBlocks<DScatter> *scattered_colblocks(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
     const int mode = env_int("SILI_COLBLOCK", 1);
-    if (mode == 0 || s.nnz == 0 || B < 2 || B > 512) return 0;
+    if (mode == 0 || s.nnz == 0 || B < 2 || B > 512) return nullptr;
     const int64_t opbytes = s.cols * B * 4;
-    if (opbytes <= (int64_t(4) << 20) || opbytes >= (int64_t)0x80000000LL) return 0;
+    if (opbytes <= (int64_t(4) << 20) || opbytes >= (int64_t)0x80000000LL) return nullptr;
     const int64_t slice = (int64_t)std::max(1, env_int("SILI_COLBLOCK_MB", 2)) << 20;
     const int64_t K = std::min<int64_t>(16, (opbytes + slice - 1) / slice);
-    return K < 2 ? 0 : K;
+    return K < 2 ? nullptr : colblocks(L, s, K, (s.cols + K - 1) / K, st);
 }
 
-bool gather_colblocked(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t B, float *out,
+void gather_colblocked(const ColBlocks<DScatter> &c, const ScaleView &sc, const float *in, int64_t B, float *out,
                        int64_t out_ld, int skip, hipStream_t st) {
-    const int64_t K = colblock_passes(s, in, B);
-    if (K == 0) return false;
-    const int64_t cb = (s.cols + K - 1) / K;
-    if ((int64_t)s.cblk.size() != K || s.cblk_cb != cb) build_colblocks(L, s, (int)K, cb);
-    else if (s.cblk_stale) refresh_colblocks(s, st);
-    for (int64_t k = 0; k < K; ++k) {
-        DScatter &sub = s.cblk[(size_t)k];
-        const int64_t c0 = k * cb;
+    for (size_t k = 0; k < c.block.size(); ++k) {
+        const DScatter &sub = c.block[k];
+        const int64_t c0 = (int64_t)k * c.width;
         const ScaleView sk{sc.row, sc.ent ? sc.ent + c0 * sc.rank : nullptr, sc.rank};
         // pass 0 stores (split rows zeroed first), later passes add
         if (k == 0) launch_zero_split_rows(sub.plan(), out, out_ld, B, st);
         launch_gather(sub.plan(), sk, in + c0 * B, B, out, out_ld, B, skip, st, k > 0);
     }
-    return true;
 }
 
 bool gather_b4_colblocked(Layer &L, DBlock4 &b, const ScaleView &sc, const float *in, int64_t B, float *out,
@@ -464,12 +457,12 @@ bool gather_b4_colblocked(Layer &L, DBlock4 &b, const ScaleView &sc, const float
     const int64_t K = std::min<int64_t>(16, (opbytes + slice - 1) / slice);
     if (K < 2) return false;
     const int64_t cbb = (b.bcols + K - 1) / K;
-    if ((int64_t)b.cblk.size() != K || b.cblk_cbb != cbb) build_colblocks_b4(L, b, (int)K, cbb);
-    else if (b.cblk_stale) refresh_colblocks_b4(b, st);
+    const ColBlocks<DBlock4> *c = colblocks(L, b, K, cbb, st);
+    if (!c) return false;
     for (int64_t k = 0; k < K; ++k) {
         const int64_t c0 = k * cbb * 4;
         const ScaleView sk{sc.row, sc.ent ? sc.ent + c0 * sc.rank : nullptr, sc.rank};
-        launch_gather_b4(b.cblk[(size_t)k].plan(), sk, in + c0 * B, B, out, out_ld, B, skip, st);
+        launch_gather_b4(c->block[(size_t)k].plan(), sk, in + c0 * B, B, out, out_ld, B, skip, st);
     }
     return true;
 }
@@ -496,16 +489,16 @@ void forward_dense(Layer &L, const float *x, int64_t B, float *y, hipStream_t st
     const bool str = L.Wt.nnz > 0 && !m24 && stream_wanted(L.Wt, ssc, B, B, skip);
     // batches 65..128: the input staged in LDS slice by slice
     const bool staged = L.Wt.nnz > 0 && !m24 && !str && staged_supported(L, L.Wt, ssc, xT, B, skip) && staged_wanted(L.Wt, B);
-    const bool plain = L.Wt.nnz > 0 && !m24 && !str && !staged && colblock_passes(L.Wt, xT, B) == 0;
+    const ColBlocks<DScatter> *cb = m24 || str || staged ? nullptr : scattered_colblocks(L, L.Wt, B, st);
+    const bool plain = L.Wt.nnz > 0 && !m24 && !str && !staged && !cb;
     if (L.Wt.nnz == 0) prep.fill(y, B * L.n_out, 0.0f);
     else if (plain) prep.zero_split(L.Wt.plan(), y, L.n_out, B);
     prep.run();
     if (m24) launch_mfma24(L, L.Wt, ssc, x, L.n_in, xT, L.ws_xT.p, B, y, L.n_out, st);
     else if (str) stream_gather(L, L.Wt, ssc, xT, B, y, L.n_out, st);
     else if (staged) launch_gather_staged(L, L.Wt, ssc, xT, B, y, L.n_out, st);
+    else if (cb) gather_colblocked(*cb, ssc, xT, B, y, L.n_out, skip, st);
     else if (plain) launch_gather(gather_plan(L, L.Wt, B), ssc, xT, B, y, L.n_out, B, skip, st);
-    else if (L.Wt.nnz > 0 && !gather_colblocked(L, L.Wt, ssc, xT, B, y, L.n_out, skip, st))
-        throw_error(SILI_ERR_RUNTIME, "forward_dense: column-block passes did not apply (internal error)");
     if (L.B4t.ntiles > 0 && !gather_b4_colblocked(L, L.B4t, shadow_scales(L), xT, B, y, L.n_out, SKIP_NONE, st))
         launch_gather_b4(L.B4t.plan(), shadow_scales(L), xT, B, y, L.n_out, B, SKIP_NONE, st);
 }
@@ -597,8 +590,11 @@ void backward_dense(Layer &L, const float *x, const float *dy, int64_t B, float 
                        launch_bwd_fused(L.W.plan(), canon_scales(L), gT, xT, B, dx, L.n_in, gw_s, L.acc_in.p, st);
     if (m24) launch_mfma24(L, L.W, canon_scales(L), dy, L.n_out, gT, nullptr, B, dx, L.n_in, st);
     else if (str) stream_gather(L, L.W, canon_scales(L), gT, B, dx, L.n_in, st);
-    else if (scat && !fused && !gather_colblocked(L, L.W, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st))
-        launch_gather(gather_plan(L, L.W, B), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
+    else if (scat && !fused) {
+        if (const ColBlocks<DScatter> *cb = scattered_colblocks(L, L.W, B, st))
+            gather_colblocked(*cb, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st);
+        else launch_gather(gather_plan(L, L.W, B), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
+    }
     if (L.B4.ntiles > 0 && !gather_b4_colblocked(L, L.B4, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st))
         launch_gather_b4(L.B4.plan(), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
     if (scat && gw_s && !fused) launch_sddmm(L.W.plan(), xT, gT, B, gw_s, L.acc_in.p, st);
@@ -703,11 +699,8 @@ void backward_dense_train(Layer &L, const float *x, const float *dy, int64_t B, 
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
         sc->drop_m24();
-        sc->values_changed();
     }
-    for (DBlock4 *b4 : {&L.B4, &L.B4t}) {
-        b4->cblk_stale = true;
-    }
+    colblock_values_changed(L, st);
     L.vs_ones = false;
     if (L.output_scale_trainable && scales_step) L.os_ones = false;
     ++L.train_calls;
@@ -792,11 +785,8 @@ void backward_sparse_train(Layer &L, const float *x, const int32_t *dptrs, const
     for (DScatter *sc : {&L.W, &L.Wt}) {
         sc->stream1.valid = sc->streamK.valid = false;
         sc->drop_m24();
-        sc->values_changed();
     }
-    for (DBlock4 *b4 : {&L.B4, &L.B4t}) {
-        b4->cblk_stale = true;
-    }
+    colblock_values_changed(L, st);
     L.vs_ones = false;
     ++L.train_calls;
     ++L.rng_calls;

@@ -95,6 +95,21 @@ struct DFor {
     DevBuf<uint8_t> bytes;
 };
 
+// Column-block copies of a store, for gathers whose operand exceeds one XCD's
+// L2: block[k] holds every row's entries with (block) columns in [k*width,
+// (k+1)*width), columns relative to the block.  An update changes values, not
+// places: a block keeps its entries' places in the store (from) and takes the
+// new values on its next use (stale), where building it anew costs a decode and
+// a scan and an encoding per block.  captured: a stream capture has recorded
+// these buffers, so they live until the structure changes, and an update
+// refreshes them at once.
+template <typename Store>
+struct ColBlocks {
+    std::vector<Store> block;
+    int64_t width = 0;
+    bool stale = false, captured = false;
+};
+
 // One orientation of the scattered store.
 struct DScatter {
     int64_t rows = 0, cols = 0, nnz = 0, nbytes = 0, nseg = 0;
@@ -141,23 +156,10 @@ struct DScatter {
         m24_saved = 0;
         m24_warm.reset();
     }
-    // column-block copies for gathers whose operand exceeds one XCD's L2:
-    // cblk[k] holds every row's entries with columns in [k*cblk_cb, ...),
-    // columns relative to the block (built on first use)
-    std::vector<DScatter> cblk;
-    int64_t cblk_cb = 0;
-    // an update changes values, not places: a copy keeps its entries' places in
-    // the store (from) and takes the new values on its next use (cblk_stale),
-    // where building it anew costs a decode, K scans and K encodings
+    // column-block copies: the ones last used, and captured ones; a block's
+    // entries' places in this store (built for a layer that trains)
+    std::vector<ColBlocks<DScatter>> cblk;
     DevBuf<uint32_t> from;
-    bool cblk_stale = false;
-    void values_changed() {
-        cblk_stale = true;
-        if (!cblk.empty() && !cblk[0].from.p) {
-            cblk.clear();
-            cblk_cb = 0;
-        }
-    }
     // split rows combined in item order by the float4 gather: arrivals per
     // row (rows+1, zero between launches) and per-item partial sums
     // (part_cap floats; empty: combined by atomics)
@@ -198,11 +200,9 @@ struct DBlock4 {
     // the dense 16 bytes and packs on export)
     DevBuf<uint8_t> sparse;
     DevBuf<SegDesc> seg;
-    // column-block copies (as DScatter::cblk, in block columns of cblk_cbb)
-    std::vector<DBlock4> cblk;
-    int64_t cblk_cbb = 0;
+    // column-block copies (as DScatter::cblk, in block columns)
+    std::vector<ColBlocks<DBlock4>> cblk;
     DevBuf<uint32_t> from;  // (as DScatter::from: tiles)
-    bool cblk_stale = false;
     // the tiles by column range (built on first use, kept until the structure
     // changes): each tile's block column, and for range x of rng_k and block
     // row br the first tile of the row in that range, rng_start[x*brows + br]
@@ -689,12 +689,21 @@ void device_sort_pairs_u32(Layer &L, const uint32_t *kin, uint32_t *kout, const 
 void device_sort_pairs_u64(Layer &L, const uint64_t *kin, uint64_t *kout, const uint32_t *vin,
                            uint32_t *vout, int64_t n, int bits);
 
-// Column-block copies of s (s.cblk, K blocks of cb columns; block4: cbb
-// block columns).
-void refresh_colblocks(DScatter &s, hipStream_t st);
-void refresh_colblocks_b4(DBlock4 &s, hipStream_t st);
-void build_colblocks(Layer &L, DScatter &s, int K, int64_t cb);
-void build_colblocks_b4(Layer &L, DBlock4 &b, int K, int64_t cbb);
+// Whether a capture is recording what is issued on st: such work has not run
+// when the call returns, and nothing can be waited for.
+inline bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SILI_HIP(hipStreamIsCapturing(st, &cap));
+    return cap != hipStreamCaptureStatusNone;
+}
+
+// The copies of s in K blocks of width (block) columns, holding the store's
+// values as of now on st: built or refreshed where they are not at hand, which
+// under stream capture they have to be (else NULL).
+const ColBlocks<DScatter> *colblocks(Layer &L, DScatter &s, int64_t K, int64_t width, hipStream_t st);
+const ColBlocks<DBlock4> *colblocks(Layer &L, DBlock4 &s, int64_t K, int64_t width, hipStream_t st);
+// After an update on st: the copies of L's stores no longer hold their values.
+void colblock_values_changed(Layer &L, hipStream_t st);
 // The staged-input gather (staged.hip): whether it takes this case, and
 // out[b, r] for every row r of s (written, not added).
 bool staged_supported(const Layer &L, const DScatter &s, const ScaleView &sc, const float *in, int64_t B, int skip);
@@ -716,15 +725,16 @@ void launch_mfma24(Layer &L, DScatter &s, const ScaleView &sc, const float *in, 
 // b.rng_* for K column ranges of ceil(bcols / K) block columns.
 void ensure_col_ranges(Layer &L, DBlock4 &b, int K);
 // Block4 contribution (added into out) in column-block passes when the
-// gathered operand exceeds 4 MiB (slices of SILI_COLBLOCK_B4_MB, default 8);
-// false: not applicable (then use launch_gather_b4).
+// gathered operand exceeds 4 MiB (slices of SILI_COLBLOCK_B4_MB, default 8)
+// and the copies can be had (colblocks); false: then use launch_gather_b4.
 bool gather_b4_colblocked(Layer &L, DBlock4 &b, const ScaleView &sc, const float *in, int64_t B, float *out,
                           int64_t out_ld, int skip, hipStream_t st);
-// out[b*out_ld + row] for b < B over s, in column-block passes when the
-// gathered operand (s.cols x B fp32) exceeds one XCD's L2 (pass 0 stores, the
-// others add; SILI_COLBLOCK=0 disables).  Returns false, launching nothing,
-// when the passes do not apply (then use launch_gather).
-bool gather_colblocked(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t B, float *out,
+// The copies for column-block passes over s, which apply when the gathered
+// operand (s.cols x B fp32) exceeds one XCD's L2 (SILI_COLBLOCK=0 disables);
+// NULL: they do not, or the copies cannot be had (then use launch_gather).
+const ColBlocks<DScatter> *scattered_colblocks(Layer &L, DScatter &s, int64_t B, hipStream_t st);
+// out[b*out_ld + row] for b < B over them (pass 0 stores, the others add).
+void gather_colblocked(const ColBlocks<DScatter> &c, const ScaleView &sc, const float *in, int64_t B, float *out,
                        int64_t out_ld, int skip, hipStream_t st);
 
 // ---- batch-1 stream kernels (stream.hip) ---------------------------------------

@@ -121,7 +121,6 @@ void requantize_code8(Layer &L) {
         sc->stream1.valid = sc->streamK.valid = false;
         sc->drop_m24();
         sc->cblk.clear();
-        sc->cblk_cb = 0;
     }
     refresh_nonfinite(L);
 }

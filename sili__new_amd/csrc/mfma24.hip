@@ -926,9 +926,7 @@ bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int sk
         s.m24_warm.set((size_t)B);
         if (!warm || (!s.m24_valid && s.m24_saved < s.m24_cost * s.m24_wait)) return false;
     }
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    SILI_HIP(hipStreamIsCapturing(st, &cap));
-    if (cap != hipStreamCaptureStatusNone) return false;
+    if (capturing(st)) return false;
     const bool built = s.m24_valid;
     if (!ensure_mfma24(L, s, B, st)) return false;
     if (mode != 2 && !built && gain() < 0) {  // the overflow entries are more than estimated

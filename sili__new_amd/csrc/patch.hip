@@ -685,7 +685,6 @@ void invalidate_derived(DScatter &s) {
     s.drop_m24();
     s.m24_failed = false;
     s.cblk.clear();
-    s.cblk_cb = 0;
 }
 
 // split_rows, n_split and has_split of s from its work items.
@@ -1173,9 +1172,7 @@ bool patch_block_row(Layer &L, const BlockRowState &old, const BlockRowState &nu
         L.B4t.ntiles += dBt.delems;
         L.B4t.nseg += dBt.dseg;
         L.B4.cblk.clear();
-        L.B4.cblk_cbb = 0;
         L.B4t.cblk.clear();
-        L.B4t.cblk_cbb = 0;
         L.B4.rng_k = L.B4t.rng_k = 0;
         if (dB.split_maybe_changed) refresh_split_b4(L, L.B4);
         if (dBt.split_maybe_changed) refresh_split_b4(L, L.B4t);
