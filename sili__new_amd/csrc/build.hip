@@ -810,9 +810,10 @@ void ensure_short_rows(Layer &L, DScatter &s) {
 }
 }  // namespace
 
-GatherPlan gather_plan(Layer &L, DScatter &s, int64_t nb) {
+GatherPlan gather_plan(Layer &L, DScatter &s, int64_t nb, hipStream_t st) {
     GatherPlan p = s.plan();
-    if (nb > 1 && nb <= SHORT_MAX_BATCH) {
+    // (the split reads a count back, which a capture does not allow)
+    if (nb > 1 && nb <= SHORT_MAX_BATCH && (s.sh_valid || !capturing(st))) {
         ensure_short_rows(L, s);
         if (s.n_sh > 0) {
             p.sh_seg = s.sh_seg.p;

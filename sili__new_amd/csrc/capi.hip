@@ -498,7 +498,7 @@ void forward_dense(Layer &L, const float *x, int64_t B, float *y, hipStream_t st
     else if (str) stream_gather(L, L.Wt, ssc, xT, B, y, L.n_out, st);
     else if (staged) launch_gather_staged(L, L.Wt, ssc, xT, B, y, L.n_out, st);
     else if (cb) gather_colblocked(*cb, ssc, xT, B, y, L.n_out, skip, st);
-    else if (plain) launch_gather(gather_plan(L, L.Wt, B), ssc, xT, B, y, L.n_out, B, skip, st);
+    else if (plain) launch_gather(gather_plan(L, L.Wt, B, st), ssc, xT, B, y, L.n_out, B, skip, st);
     if (L.B4t.ntiles > 0 && !gather_b4_colblocked(L, L.B4t, shadow_scales(L), xT, B, y, L.n_out, SKIP_NONE, st))
         launch_gather_b4(L.B4t.plan(), shadow_scales(L), xT, B, y, L.n_out, B, SKIP_NONE, st);
 }
@@ -593,7 +593,7 @@ void backward_dense(Layer &L, const float *x, const float *dy, int64_t B, float 
     else if (scat && !fused) {
         if (const ColBlocks<DScatter> *cb = scattered_colblocks(L, L.W, B, st))
             gather_colblocked(*cb, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st);
-        else launch_gather(gather_plan(L, L.W, B), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
+        else launch_gather(gather_plan(L, L.W, B, st), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
     }
     if (L.B4.ntiles > 0 && !gather_b4_colblocked(L, L.B4, canon_scales(L), gT, B, dx, L.n_in, SKIP_NONE, st))
         launch_gather_b4(L.B4.plan(), canon_scales(L), gT, B, dx, L.n_in, B, SKIP_NONE, st);
@@ -731,7 +731,7 @@ void forward_sparse(Layer &L, const int32_t *ptrs, const int32_t *idx, const flo
     const ScaleView ssc = comp0_scales(L, true, st);
     if (!push) {
         launch_zero_split_rows(L.Wt.plan(), y, L.n_out, B, st);
-        launch_gather(gather_plan(L, L.Wt, B), ssc, L.ws_xT.p, B, y, L.n_out, B, SKIP_POSZERO, st);
+        launch_gather(gather_plan(L, L.Wt, B, st), ssc, L.ws_xT.p, B, y, L.n_out, B, SKIP_POSZERO, st);
     }
     if (L.B4t.ntiles > 0) launch_gather_b4(L.B4t.plan(), ssc, L.ws_xT.p, B, y, L.n_out, B, SKIP_POSZERO, st);
 }
@@ -748,7 +748,7 @@ void backward_sparse(Layer &L, const float *x, const int32_t *dptrs, const int32
     // scattered: merge-join visits only present dy entries (sisldo_ops.hpp:705-713);
     // block4: skips dy == 0 per slot (sisldo_ops.hpp:886-897)
     const ScaleView csc = comp0_scales(L, false, st);
-    launch_gather(gather_plan(L, L.W, B), csc, L.ws_gT.p, B, dx, L.n_in, B, SKIP_POSZERO, st);
+    launch_gather(gather_plan(L, L.W, B, st), csc, L.ws_gT.p, B, dx, L.n_in, B, SKIP_POSZERO, st);
     if (L.B4.ntiles > 0) launch_gather_b4(L.B4.plan(), csc, L.ws_gT.p, B, dx, L.n_in, B, SKIP_ZERO, st);
 }
 

@@ -615,7 +615,7 @@ void dense_to_top_k_csr_device(const float *x, int64_t rows, int64_t cols, int64
 // rocprim wrappers
 // The plan of a scattered store for a float4 gather over nb batch columns:
 // with its short rows split off (built on first use) where that applies.
-GatherPlan gather_plan(Layer &L, DScatter &s, int64_t nb);
+GatherPlan gather_plan(Layer &L, DScatter &s, int64_t nb, hipStream_t st);
 void device_exclusive_scan_u64(Layer &L, const uint64_t *in, uint64_t *out, int64_t n);
 void device_exclusive_scan_u32(Layer &L, const uint32_t *in, uint32_t *out, int64_t n);
 // Small device values read back with one stream synchronization: each
