@@ -1109,6 +1109,7 @@ static const ColBlocks<Store> *find_colblocks(Layer &L, Store &s, int64_t K, int
     if (cap) return nullptr;
     s.cblk.erase(std::remove_if(s.cblk.begin(), s.cblk.end(), [](const ColBlocks<Store> &c) { return !c.captured; }),
                  s.cblk.end());
+    finish_updates(L, st);
     s.cblk.push_back(build_colblocks(L, s, K, width));
     return &s.cblk.back();
 }

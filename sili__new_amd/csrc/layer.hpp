@@ -697,6 +697,12 @@ inline bool capturing(hipStream_t st) {
     return cap != hipStreamCaptureStatusNone;
 }
 
+// Before a copy of the store's values is built on the layer's stream for a call
+// on st: an update that st still runs has to have written them.
+inline void finish_updates(const Layer &L, hipStream_t st) {
+    if (st != L.stream) SILI_HIP(hipStreamSynchronize(st));
+}
+
 // The copies of s in K blocks of width (block) columns, holding the store's
 // values as of now on st: built or refreshed where they are not at hand, which
 // under stream capture they have to be (else NULL).

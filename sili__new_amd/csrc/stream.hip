@@ -877,11 +877,15 @@ void stream_gather(Layer &L, DScatter &s, const ScaleView &sc, const float *in, 
     DStream *d = nullptr;
     if (K == 1) {
         d = &s.stream1;
-        if (!d->valid && !d->failed) build_stream(L, s, *d, 1, s.cols);
+        if (!d->valid && !d->failed) {
+            finish_updates(L, st);
+            build_stream(L, s, *d, 1, s.cols);
+        }
     } else {
         d = &s.streamK;
         if (!d->valid || d->K != K || d->cb != cb) {
             d->failed = false;
+            finish_updates(L, st);
             build_stream(L, s, *d, K, cb);
         }
     }
