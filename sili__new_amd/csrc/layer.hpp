@@ -404,8 +404,9 @@ struct Layer {
     DevBuf<float> ws_s0;  // component 0 of rank > 1 scales: value [n_in], then output [n_out]
     DevBuf<float> ws_xs;  // the staged-input gather's column-scaled input copy
     DevBuf<uint16_t> ws_m24;  // the matrix-core gather's input pieces (bf16)
-    DevBuf<int> m24_flag;     // set by its split kernel to the call's number: an input has no pieces
-    int m24_epoch = 0;
+    // per batch row: set by its split kernel to the call's number where an input has no pieces
+    DevBuf<uint32_t> m24_flag;
+    uint32_t m24_epoch = 0;
     int64_t xT_cached_batch = 0;  // > 0: ws_xT holds the last forward_dense input, feature-major
     Scratch scratch;
     Profiler prof;

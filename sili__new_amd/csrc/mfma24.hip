@@ -15,9 +15,13 @@
 //     in fp32 beforehand, the row scale to the sum, as in the staged gather);
 //   - an fp32 input is the exact sum of three bf16 pieces (8 + 8 + 8 bits), so
 //     three products with fp32 accumulation stand for the one;
-//   - inputs that have no such pieces (non-finite, or nonzero below 2^-110)
-//     are seen by the split kernel, and the whole call then takes an fp32
-//     loop over the store's synapses inside the same kernel.
+//   - inputs (times their column scale) are shifted by 2^60 before they are
+//     split, the sums back by the row scale's product: every fp32 input down to
+//     the subnormals then has its pieces in bf16's normal range, and no sum of
+//     the 2^21 columns at most overflows.  Batch rows holding an input outside
+//     that window (non-finite, or 2^42 and more) are seen by the split kernel
+//     and computed from the store's synapses by the same kernel in the order of
+//     the other gathers (code * (row scale * column scale)) * input.
 // Columns of a group of 4 beyond the second go to an overflow list (1 % of the
 // synapses at 10 % density), added in fp32 before the output is written.
 //
@@ -51,6 +55,7 @@ constexpr int64_t KB = 128;       // columns per block of the copy
 // registers go round without a branch (at which the compiler waits for every
 // load in flight).
 inline int64_t n_blocks(int64_t cols) { return ((cols + KB - 1) / KB + 3) & ~int64_t(3); }
+constexpr int64_t MAX_B = 512;    // batches that the gather serves
 constexpr int64_t BUILD_K = 4096;  // columns a build block holds in LDS (48 KiB)
 
 // ---- building the copy ---------------------------------------------------------
@@ -71,8 +76,8 @@ __device__ __forceinline__ uint32_t group_rank(const int32_t *__restrict__ cols,
     return rank;
 }
 
-__global__ void k_m24_clear(uint32_t *p) {
-    if (threadIdx.x == 0u) *p = 0u;
+__global__ void k_m24_clear(uint32_t *p, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
 }
 
 // ovf_n[r] = the row's overflow entries (codes other than 0): one wave per row.
@@ -177,17 +182,24 @@ __global__ __launch_bounds__(256) void k_m24_build(const uint32_t *__restrict__ 
 
 // ---- the input's pieces ----------------------------------------------------------
 
-// x = p[0] + p[1] + p[2] exactly, each a bf16 (round to nearest: the
-// remainders have at most 16 and 8 significant bits); false when x is not
-// finite or so small that the last piece would leave bf16's range.
-__device__ __forceinline__ bool split3(float x, __bf16 (&p)[3]) {
-    p[0] = (__bf16)x;
-    const float r1 = x - (float)p[0];
+// v = p[0] + p[1] + p[2] exactly, each a bf16 (round to nearest: the
+// remainders have at most 16 and 8 significant bits); v = x * scale.  False
+// where v is outside the window: below 2^-102 the last piece would be
+// subnormal, and 2^21 columns of 6 * 2^102 are what a sum holds.
+__device__ __forceinline__ bool split3(float x, float scale, __bf16 (&p)[3]) {
+    const float v = x * scale;
+    p[0] = (__bf16)v;
+    const float r1 = v - (float)p[0];
     p[1] = (__bf16)r1;
     p[2] = (__bf16)(r1 - (float)p[1]);
-    const float a = __builtin_fabsf(x);
-    // (a value that rounds up to bf16's infinity has no pieces either)
-    return a == 0.0f || (a >= 0x1p-110f && a < 0x1.fep127f);
+    const float a = __builtin_fabsf(v);
+    return (a == 0.0f && (x == 0.0f || scale == 0.0f)) || (a >= 0x1p-102f && a < 0x1p102f);
+}
+constexpr float SHIFT = 0x1p60f;
+// A sum of shifted terms, times the row scale (neither product leaves the
+// range on the way unless the result does).
+__device__ __forceinline__ float unshifted(float sum, float rs) {
+    return __builtin_fabsf(rs) < 1.0f / SHIFT ? (sum * rs) * (1.0f / SHIFT) : sum * (rs * (1.0f / SHIFT));
 }
 
 struct SplitArgs {
@@ -196,8 +208,8 @@ struct SplitArgs {
     const float *ent;     // column scales, or NULL
     float *xT;            // the input feature-major [cols][B] (without the scales), or NULL
     __bf16 *out;
-    int *flag;            // set to epoch, this call's number, when an input has no pieces
-    int epoch;
+    uint32_t *flag;       // per batch row: set to epoch, this call's number, when an input has no pieces
+    uint32_t epoch;
     int64_t nsteps;       // 32-column steps (a multiple of 4)
     int nt;               // column tiles of 32
 };
@@ -227,14 +239,15 @@ __global__ __launch_bounds__(256) void k_m24_split(SplitArgs a) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int64_t k = k0 + j;
-        float x = 0.0f;
+        float x = 0.0f, scale = SHIFT;
         if (on && k < a.cols) {
             x = src[k];
             if (a.xT && piece == 0) a.xT[k * a.B + b] = x;
-            if (a.ent) x *= a.ent[k];
+            if (a.ent) scale *= a.ent[k];
         }
         __bf16 p[3];
-        ok = split3(x, p) && ok;
+        // (up to 2^60, a column scale's products with the shift and a code are finite)
+        ok = split3(x, scale, p) && __builtin_fabsf(scale) <= 0x1p120f && ok;
         if constexpr (SMALL) {
             h[0][j] = piece == 0 ? p[0] : piece == 1 ? p[1] : p[2];
         } else {
@@ -242,7 +255,7 @@ __global__ __launch_bounds__(256) void k_m24_split(SplitArgs a) {
             for (int q = 0; q < 3; ++q) h[q][j] = p[q];
         }
     }
-    if (!ok) *a.flag = a.epoch;
+    if (!ok) a.flag[b] = a.epoch;
     // (as in k_transpose)
     if (a.xT && a.B % 4 != 0 && blockIdx.x == 0 && threadIdx.x < (uint32_t)BATCH_SLACK) a.xT[a.cols * a.B + threadIdx.x] = 0.0f;
     uint4 *o = reinterpret_cast<uint4 *>(a.out);
@@ -275,8 +288,8 @@ struct M24Args {
     const uint2 *ovf;
     int64_t rows, cols, nkb, ntile;
     const __bf16 *xf;           // the input's operands
-    const int *flag;            // epoch: an input of this call has no pieces
-    int epoch;
+    const uint32_t *flag;       // per batch row; epoch: an input of this call has no pieces
+    uint32_t epoch;
     const float *inT;           // feature-major input [cols][B] and its column scales (or NULL)
     const float *ent;
     const float *rs;            // row scales, or NULL
@@ -307,35 +320,78 @@ __device__ __forceinline__ f16v smfmac(bf8 A, bf16x16 Bv, f16v C, const u2 &ix) 
     return __builtin_amdgcn_smfmac_f32_32x32x32_bf16(A, Bv, C, w, 0, KS & 1);
 }
 
-// out rows [r0, r1) of batch rows [b0, b1), from the store's synapses in fp32
-// (an input without bf16 pieces): one wave, a row at a time.
-__device__ void rows_in_fp32(const M24Args &a, int64_t r0, int64_t r1, int64_t b0, int64_t b1) {
+// Whether batch row b0 + lane holds an input without pieces.
+__device__ __forceinline__ uint32_t row_flag(const M24Args &a, int64_t b0) {
+    return a.flag[min<int64_t>(b0 + lane_id(), a.B - 1)];
+}
+__device__ __forceinline__ uint64_t odd_rows(const M24Args &a, int64_t b0, uint32_t flag) {
+    return __ballot(b0 + lane_id() < a.B && flag == a.epoch);
+}
+// out rows [r0, r1) of the batch rows b0 + (bits of todo), from the store's
+// synapses in fp32: one wave, a lane per synapse of a 64-byte window, 4
+// neighbouring batch rows a turn (one load a synapse for them; the others of
+// the 4 are not written).  R rows go side by side, without a branch between
+// their loads: a row alone is a chain of a window's bytes, its values and its
+// inputs.  At 5120 x 204800, 10 %, a call holding one such batch row took 1.25 ms
+// at batch 128 (0.52 without; the segment gather 1.4) and 0.97 at batch 8 (0.10;
+// the stream kernels 0.14), one holding nothing else 20 and 1.7 ms.  (A whole
+// call's loop over the batch columns instead, wherever one input was below
+// 2^-110, not finite or too large: 32 and 9.3 ms.)
+__device__ __forceinline__ void rows_in_fp32(const M24Args &a, int64_t r0, int64_t r1, int64_t b0, uint64_t todo) {
+    constexpr int R = 4;
     const uint32_t lane = lane_id();
-    for (int64_t r = r0; r < r1; ++r) {
-        const float f = a.rs ? a.rs[r] : 1.0f;
-        for (int64_t bb = b0; bb < b1; bb += 64) {
-            const int64_t b = bb + lane;
-            const bool on = b < b1;
-            float acc = 0.0f;
-            uint32_t pos = a.byte_start[r], carry = 0, ebase = a.elem_start[r];
-            const uint32_t end = a.byte_start[r + 1];
-            while (pos < end) {
-                const Chunk ch = decode_chunk(a.sidx, pos, end, carry);
-                if (ch.T == 0ull) break;
-                const uint32_t code = ch.term ? (uint32_t)(a.sval[ebase + ch.rank] >> 4) : 0u;
-                uint64_t T = ch.T;
-                while (T) {
-                    const int l = __builtin_ctzll(T);
-                    T &= T - 1ull;
-                    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)ch.col, l);
-                    const float w = fp4_decode((uint32_t)__builtin_amdgcn_readlane((int)code, l));
-                    float x = on ? a.inT[(int64_t)c * a.B + b] : 0.0f;
-                    if (a.ent) x *= a.ent[c];
-                    acc = __builtin_fmaf(w, x, acc);
-                }
-                carry = chunk_advance(ch, pos, ebase);
+    for (; todo; todo >>= 4, b0 += 4) {
+        if ((todo & 15ull) == 0ull) continue;
+        for (int64_t r = r0; r < r1; r += R) {
+            float f[R];
+            float4 acc[R];
+            uint32_t pos[R], end[R], ebase[R], carry[R];
+            bool more = false;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {  // past the last row: an empty one
+                const int64_t row = min<int64_t>(r + q, r1 - 1);
+                f[q] = a.rs ? a.rs[row] : 1.0f;
+                pos[q] = a.byte_start[row];
+                end[q] = r + q < r1 ? a.byte_start[row + 1] : pos[q];
+                ebase[q] = a.elem_start[row];
+                carry[q] = 0;
+                more = more || pos[q] < end[q];
+                acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             }
-            if (on) a.out[b * a.out_ld + r] = acc * f;
+            while (more) {
+                uint32_t byte[R];
+                Chunk ch[R];
+                float w[R];
+                float4 x[R];
+                // (a lane without a byte or a synapse loads what another one does)
+#pragma unroll
+                for (int q = 0; q < R; ++q) byte[q] = a.sidx[pos[q] + lane < end[q] ? pos[q] + lane : 0u];
+#pragma unroll
+                for (int q = 0; q < R; ++q) ch[q] = decode_window(pos[q] + lane < end[q] ? byte[q] : 0x80u, carry[q]);
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                    w[q] = fp4_decode((uint32_t)(a.sval[ch[q].term ? ebase[q] + ch[q].rank : 0u] >> 4)) *
+                           (a.ent ? f[q] * a.ent[ch[q].col] : f[q]);
+                    x[q] = load_f4(a.inT + (uint64_t)ch[q].col * (uint32_t)a.B + b0);  // (3 floats past the last input at most)
+                }
+                more = false;
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                    acc[q].x = ch[q].term ? __builtin_fmaf(w[q], x[q].x, acc[q].x) : acc[q].x;
+                    acc[q].y = ch[q].term ? __builtin_fmaf(w[q], x[q].y, acc[q].y) : acc[q].y;
+                    acc[q].z = ch[q].term ? __builtin_fmaf(w[q], x[q].z, acc[q].z) : acc[q].z;
+                    acc[q].w = ch[q].term ? __builtin_fmaf(w[q], x[q].w, acc[q].w) : acc[q].w;
+                    if (ch[q].T == 0ull) pos[q] = end[q];
+                    else carry[q] = chunk_advance(ch[q], pos[q], ebase[q]);
+                    more = more || pos[q] < end[q];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const float4 sum = make_float4(wave_sum(acc[q].x), wave_sum(acc[q].y), wave_sum(acc[q].z), wave_sum(acc[q].w));
+                if (lane < 4u && ((todo >> lane) & 1ull) && r + q < r1)
+                    a.out[(b0 + lane) * a.out_ld + r + q] = lane < 2u ? (lane == 0u ? sum.x : sum.y) : (lane == 2u ? sum.z : sum.w);
+            }
         }
     }
 }
@@ -449,7 +505,7 @@ __device__ __forceinline__ void add_overflow(const M24Args &a, float *col, uint3
     for (uint32_t o = o0; o < o1; o += 64u) {
         const uint32_t n = min(64u, o1 - o);
         const uint2 e = a.ovf[min(o + lane, o1 - 1u)];
-        float w = __builtin_bit_cast(float, e.y);
+        float w = __builtin_bit_cast(float, e.y) * SHIFT;
         if constexpr (ENT) w *= a.ent[e.x & 0x7FFFFFu];
         for (uint32_t j = 0; j < n; j += U) {
             float v[U][C], we[U];
@@ -513,11 +569,8 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t lane = lane_id(), wave = uniform(threadIdx.x >> 6), wm = wave / WN, wn = wave % WN;
     const int64_t tile0 = ((int64_t)blockIdx.x * WM + wm) * MT;
-    const int64_t n0 = (int64_t)blockIdx.y * 128 + wn * 32;
-    if (*a.flag == a.epoch) {
-        rows_in_fp32(a, tile0 * 32, min<int64_t>(a.rows, (tile0 + MT) * 32), n0, min<int64_t>(a.B, n0 + 32));
-        return;
-    }
+    const int64_t b0 = (int64_t)blockIdx.y * 128;
+    const uint32_t flag0 = row_flag(a, b0), flag1 = WN == 4 ? row_flag(a, b0 + 64) : 0u;
     const uint32_t nstages = (uint32_t)a.nkb * WN;
     const __amdgpu_buffer_rsrc_t xf = buffer_rsrc(
         reinterpret_cast<const uint8_t *>(a.xf) + (int64_t)blockIdx.y * 4 * 3 * a.nkb * 4 * 2048, nstages * STAGE);
@@ -546,6 +599,7 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
     stage(0);
     stage(1);
     landed_for_block<0>();
+    const uint64_t odd0 = odd_rows(a, b0, flag0), odd1 = WN == 4 ? odd_rows(a, b0 + 64, flag1) : 0ull;
     const uint32_t bs0 = lds_address(lds) + wn * 2048u + lane * 16u;
     auto block = [&](auto slot, uint32_t kb) {
         constexpr int R = decltype(slot)::value;
@@ -585,7 +639,7 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) tile_to_lds(s + wn * 32 * LD + (wm * MT + i) * 32, LD, hi[i] + lo[i]);
     __syncthreads();
-    const int64_t b0 = (int64_t)blockIdx.y * 128, r0 = (int64_t)blockIdx.x * R;
+    const int64_t r0 = (int64_t)blockIdx.x * R;
     const uint32_t nb = (uint32_t)min<int64_t>(a.B - b0, 32 * WN);
     {
         constexpr int C = WN == 4 ? 2 : 1;
@@ -606,7 +660,12 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
         const float f = a.rs ? a.rs[r0 + m] : 1.0f;
         float *out = a.out + b0 * a.out_ld + r0 + m;
 #pragma unroll 4
-        for (uint32_t b = wave; b < nb; b += 8u) out[b * a.out_ld] = s[b * LD + m] * f;
+        for (uint32_t b = wave; b < nb; b += 8u) out[b * a.out_ld] = unshifted(s[b * LD + m], f);
+    }
+    if (odd0 | odd1) {
+        __syncthreads();  // (over what was written above)
+        const int64_t w0 = min<int64_t>(r0 + wave * RW, a.rows), w1 = min<int64_t>(w0 + RW, a.rows);
+        for (int h = 0; h < 2; ++h) rows_in_fp32(a, w0, w1, b0 + 64 * h, h ? odd1 : odd0);
     }
 }
 
@@ -620,7 +679,7 @@ constexpr int SMALL_B = 21;
 // entries of a row by the two lanes that hold it (half h: batch rows [h
 // ceil(B/2), ...)).
 template <int Q, bool ENT>  // Q: batch rows per lane at most, a multiple of 4
-__device__ __forceinline__ void write_rows_small(const M24Args &a, const float *s, int64_t tile) {
+__device__ __forceinline__ void write_rows_small(const M24Args &a, const float *s, int64_t tile, uint32_t odd) {
     constexpr uint32_t LD = 33u;
     constexpr int U = 4;
     const uint32_t lane = lane_id(), half = lane >> 5, m = lane & 31u;
@@ -645,7 +704,7 @@ __device__ __forceinline__ void write_rows_small(const M24Args &a, const float *
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             const uint32_t k = next[i].x & 0x7FFFFFu;
-            w[i] = __builtin_bit_cast(float, next[i].y);
+            w[i] = __builtin_bit_cast(float, next[i].y) * SHIFT;
             if constexpr (ENT) w[i] *= a.ent[k];
 #pragma unroll
             for (int q = 0; q < Q / 4; ++q)  // (reads up to Q floats from b0: the input's buffer is padded by 64 bytes)
@@ -666,22 +725,18 @@ __device__ __forceinline__ void write_rows_small(const M24Args &a, const float *
     const float f = a.rs && r < a.rows ? a.rs[r] : 1.0f;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-        if (b0 + q < b1 && r < a.rows) a.out[(int64_t)(b0 + q) * a.out_ld + r] = y[q] * f;
+        if (b0 + q < b1 && r < a.rows && !((odd >> (b0 + q)) & 1u)) a.out[(int64_t)(b0 + q) * a.out_ld + r] = unshifted(y[q], f);
     wave_lds_sync();
 }
 
 constexpr int RING = 4;
 template <int MT, int NT>
-__global__ __launch_bounds__(256, 2) void k_m24_small(M24Args a) {
+__global__ __launch_bounds__(256, NT == 1 ? 4 : 2) void k_m24_small(M24Args a) {
     constexpr uint32_t STEP = NT * 2048u, STAGE = 4 * STEP;  // bytes
     constexpr int DOPS = STAGE / 4096, AOPS = 2 * MT, AHEAD = 3;
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t lane = lane_id(), wave = uniform(threadIdx.x >> 6);
     const int64_t tile0 = ((int64_t)blockIdx.x * 4 + wave) * MT;
-    if (*a.flag == a.epoch) {
-        rows_in_fp32(a, tile0 * 32, min<int64_t>(a.rows, (tile0 + MT) * 32), 0, a.B);
-        return;
-    }
     const __amdgpu_buffer_rsrc_t xf = buffer_rsrc(a.xf, (uint32_t)a.nkb * STAGE);
     auto stage = [&](uint32_t t) {
         const uint32_t at = (t & (RING - 1)) * STAGE + wave * 1024u;
@@ -741,6 +796,7 @@ __global__ __launch_bounds__(256, 2) void k_m24_small(M24Args a) {
         block(std::integral_constant<int, 3>{}, kb + 3);
     }
     landed_for_block<0>();
+    const uint32_t odd = (uint32_t)odd_rows(a, 0, row_flag(a, 0));  // (B <= SMALL_B)
     float *s = reinterpret_cast<float *>(lds) + wave * (NT * 32 * 33u);
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -748,13 +804,14 @@ __global__ __launch_bounds__(256, 2) void k_m24_small(M24Args a) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) tile_to_lds(s + j * 32 * 33u, 33u, acc[i][j]);
         if (NT == 1 && a.B <= 8) {
-            if (a.ent) write_rows_small<4, true>(a, s, tile0 + i);
-            else write_rows_small<4, false>(a, s, tile0 + i);
+            if (a.ent) write_rows_small<4, true>(a, s, tile0 + i, odd);
+            else write_rows_small<4, false>(a, s, tile0 + i, odd);
         } else {
-            if (a.ent) write_rows_small<NT == 1 ? 8 : 12, true>(a, s, tile0 + i);
-            else write_rows_small<NT == 1 ? 8 : 12, false>(a, s, tile0 + i);
+            if (a.ent) write_rows_small<NT == 1 ? 8 : 12, true>(a, s, tile0 + i, odd);
+            else write_rows_small<NT == 1 ? 8 : 12, false>(a, s, tile0 + i, odd);
         }
     }
+    if (odd) rows_in_fp32(a, min<int64_t>(a.rows, tile0 * 32), min<int64_t>(a.rows, (tile0 + MT) * 32), 0, odd);
 }
 
 // Operand column tiles of a batch (of its pieces, up to SMALL_B).
@@ -852,8 +909,8 @@ static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
     try {
         L.ws_m24.ensure(ops);
         if (!L.m24_flag.p) {
-            L.m24_flag.ensure(1);
-            launch(k_m24_clear, dim3(1), dim3(64), 0, st, reinterpret_cast<uint32_t *>(L.m24_flag.p));
+            L.m24_flag.ensure(MAX_B);
+            launch(k_m24_clear, dim3(1), dim3(64), 0, st, L.m24_flag.p, (uint32_t)MAX_B);
             L.m24_epoch = 0;
         }
         if (s.m24_valid) return true;
@@ -865,7 +922,7 @@ static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
         DevBuf<uint32_t> cnt;
         cols.ensure((size_t)s.nnz + 1);
         cnt.ensure((size_t)s.rows + 2);  // the scan's, and the most of a row
-        launch(k_m24_clear, dim3(1), dim3(64), 0, st, cnt.p + s.rows + 1);
+        launch(k_m24_clear, dim3(1), dim3(64), 0, st, cnt.p + s.rows + 1, 1u);
         launch_decode(s.plan(), ScaleView{nullptr, nullptr, 1}, cols.p, nullptr, nullptr, st);
         const dim3 rgrid((unsigned)((s.rows + 3) / 4));
         launch(k_m24_count, rgrid, dim3(TPB), 0, st, (const uint32_t *)s.elem_start.p, (const int32_t *)cols.p,
@@ -912,7 +969,7 @@ bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int sk
     // (default) by the estimates
     const int mode = env_int("SILI_MFMA24", 1);
     if (mode == 0 || s.nnz == 0 || s.m24_failed || L.has_nonfinite || skip != SKIP_NONE || sc.rank != 1) return false;
-    if (B < 2 || B > 512 || s.cols > (int64_t(1) << 21)) return false;
+    if (B < 2 || B > MAX_B || s.cols > (int64_t(1) << 21)) return false;
     const double other = others_us(s, B);
     const auto gain = [&] { return 0.9 * other - mfma24_us(Shape(s), B); };
     if (mode != 2) {
@@ -942,7 +999,7 @@ void launch_mfma24(Layer &L, DScatter &s, const ScaleView &sc, const float *in, 
     const bool small = B <= SMALL_B;
     const int nt = operand_tiles(B);
     const int64_t chunks = small ? 1 : (nt + 3) / 4;
-    const int epoch = ++L.m24_epoch;
+    const uint32_t epoch = ++L.m24_epoch;
     {
         ProfScope ps("mfma24_split", st);
         const SplitArgs a{in, in_ld, s.cols, B, sc.ent, xT, reinterpret_cast<__bf16 *>(L.ws_m24.p), L.m24_flag.p, epoch,

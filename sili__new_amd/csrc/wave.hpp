@@ -147,12 +147,10 @@ struct Chunk {
     bool term;
 };
 
-__device__ __forceinline__ Chunk decode_chunk(const uint8_t *__restrict__ idx, uint32_t pos,
-                                              uint32_t end, uint32_t carry) {
+// (b: the lane's byte of the window, 0x80 past the end)
+__device__ __forceinline__ Chunk decode_window(uint32_t b, uint32_t carry) {
     Chunk ch;
     const uint32_t lane = lane_id();
-    const uint32_t p = pos + lane;
-    const uint32_t b = (p < end) ? (uint32_t)idx[p] : 0x80u;
     const bool term = (b & 0x80u) == 0u;
     const uint64_t T = __ballot(term);
     // continuation flags of the 4 bytes before this lane, bit 3 = lane-1; the
@@ -180,6 +178,11 @@ __device__ __forceinline__ Chunk decode_chunk(const uint8_t *__restrict__ idx, u
     ch.term = term;
     ch.T = T;
     return ch;
+}
+__device__ __forceinline__ Chunk decode_chunk(const uint8_t *__restrict__ idx, uint32_t pos,
+                                              uint32_t end, uint32_t carry) {
+    const uint32_t p = pos + lane_id();
+    return decode_window((p < end) ? (uint32_t)idx[p] : 0x80u, carry);
 }
 
 // Advance a decoder past a window: returns the new carry (column of the

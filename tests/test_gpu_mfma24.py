@@ -103,6 +103,62 @@ def test_mfma24_inputs_without_a_split(hip, monkeypatch, kind, B):
     check(hip, H, L, *fine, f"after {kind} B{B}")
 
 
+@pytest.mark.parametrize("B", [8, 16, 37, 64, 150])
+@pytest.mark.parametrize("kind", ["large x", "large dy", "scales", "octaves", "zero scales"])
+def test_mfma24_ranges(hip, monkeypatch, kind, B):
+    """Finite results whose way there could leave the range: inputs near the
+    largest float under small scales, scales that cancel each other, batch rows
+    of every magnitude down to the subnormals, scales of 0."""
+    monkeypatch.setenv("SILI_MFMA24", "2")
+    H, L = make(hip, 300, 400, 0.2, 5, False)
+    rng = np.random.default_rng(B)
+    x, dy = rng.normal(size=(B, 300)).astype(np.float32), rng.normal(size=(B, 400)).astype(np.float32)
+    vs, os_ = rng.uniform(0.5, 1.5, 300).astype(np.float32), rng.uniform(0.5, 1.5, 400).astype(np.float32)
+    if kind == "large x":  # sums of up to 300 terms of 6 * 3e37 * 0.007 at most, larger by 1 / 0.003 without the output's scale
+        x[::3] = rng.uniform(-3e37, 3e37, x[::3].shape)
+        x[0, 3], os_ = 0.0, os_ * np.float32(0.003)
+    elif kind == "large dy":
+        dy[1::3] = rng.uniform(-3e37, 3e37, dy[1::3].shape)
+        dy[1, 3], vs = -0.0, vs * np.float32(0.003)
+    elif kind == "scales":  # an input times its own scale alone is subnormal, or infinite
+        x, dy = x * np.float32(1e-15), dy * np.float32(1e15)
+        vs, os_ = vs * np.float32(1e-27), os_ * np.float32(1e27)
+    elif kind == "octaves":
+        x = np.ldexp(x, np.linspace(-146, 60, B).astype(int)[:, None]).astype(np.float32)
+        dy = np.ldexp(dy, np.linspace(-146, 60, B).astype(int)[:, None]).astype(np.float32)
+    else:
+        vs[::2], os_[::3] = 0.0, 0.0
+    H.set_scales(vs, os_)
+    L.set_value_scales(vs)
+    L.set_output_scales(os_)
+    got = check(hip, H, L, x, dy, f"{kind} B{B}")
+    assert all(np.all(np.isfinite(v)) for v in got.values())
+    for k, want, bound in (("y", H.forward_dense(x), H.forward_dense(x, absmode=True)),
+                           ("dx", H.backward_dense(x, dy)[0], H.backward_dense(x, dy, absmode=True)[0])):
+        # sums of n <= 400 terms: half an ulp each for the weight's two products, the input's and the
+        # sum's on either side, and a step of the subnormals
+        lim = 400 * 4 * (2.0 ** -24 * bound.astype(np.float64) + 2.0 ** -149)
+        assert np.all(np.abs(got[k].astype(np.float64) - want) <= lim), k
+
+
+@pytest.mark.parametrize("B", [8, 37, 150])
+def test_mfma24_one_row_without_a_split(hip, monkeypatch, B):
+    """Only the batch row that holds the input leaves the products: the others'
+    outputs are the same bits as without it."""
+    monkeypatch.setenv("SILI_MFMA24", "2")
+    H, L = make(hip, 300, 400, 0.2, 5, True)
+    rng = np.random.default_rng(B)
+    x, dy = rng.normal(size=(B, 300)).astype(np.float32), rng.normal(size=(B, 400)).astype(np.float32)
+    fine = check(hip, H, L, x, dy, f"fine B{B}")
+    row = B // 2
+    x[row, 17], dy[row, 20] = np.inf, np.nan
+    got = check(hip, H, L, x, dy, f"one row B{B}")
+    for k in got:
+        others = np.arange(B) != row
+        assert np.array_equal(got[k][others].view(np.uint32), fine[k][others].view(np.uint32)), k
+        assert not np.all(np.isfinite(got[k][row])), k
+
+
 def test_mfma24_copy_follows_changes(hip, monkeypatch):
     monkeypatch.setenv("SILI_MFMA24", "2")
     L = make(hip, 700, 1000, 0.1, 3, True)[1]
