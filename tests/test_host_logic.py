@@ -80,6 +80,31 @@ def test_algorithmic_bytes_table():
     assert t["bwd:gather_gradw"] == base + 4 * 8 * 32 + 2 * 4 * 8 * 64 + 4 * 1000
 
 
+def test_bench_names_the_gather_of_any_kernel():
+    sys.path.insert(0, ROOT)
+    import bench
+    # every layer on the matrix cores: no scope of the other gathers
+    kern = {"q:fwd:mfma24_split": 0.02, "q:fwd:mfma24": 0.4, "up:fwd:mfma24_split": 0.9, "up:fwd:mfma24": 0.6}
+    assert bench.dominant_gather(kern) == ("up:fwd:mfma24", 0.6)
+    assert bench.dominant_gather({"q:fwd:stream": 0.1, "up:fwd:gather": 0.3, "up:fwd:stream_zero": 0.7}) == ("up:fwd:gather", 0.3)
+    assert bench.dominant_gather({"q:fwd:another": 0.1})[0] == "q:fwd:another"
+
+
+def test_bench_warms_up_until_the_kernels_stay():
+    sys.path.insert(0, ROOT)
+    import bench
+    calls = []
+
+    def scopes():  # other kernels until the 60th step, a build in it, the matrix cores from then on
+        calls.append(1)
+        n = len(calls)
+        return {"gather"} if n < 60 else {"mfma24_build", "mfma24"} if n == 60 else {"mfma24"}
+    got, n = bench.warm_until_settled(lambda: calls.append(1), scopes)
+    assert got == {"mfma24"} and n == len(calls) and n > 60 + 100
+    flip = []
+    assert bench.warm_until_settled(lambda: None, lambda: flip.append(1) or {len(flip)}, most=200)[1] <= 221  # ends
+
+
 def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True, timeout=120)
