@@ -747,7 +747,8 @@ __global__ void k_clear_u32(uint32_t *__restrict__ p, int64_t n) {
 // wider pass, combines with atomics).
 void prepare_split_combine(Layer &L, DScatter &s) {
     const int64_t cap = s.nseg * 128;
-    if (!s.has_split || s.nseg == 0 || cap > ((int64_t)16 << 20) || env_int("SILI_SPLIT_COMBINE", 0) == 0) {
+    s.repeatable = env_int("SILI_SPLIT_COMBINE", 0) != 0;
+    if (!s.has_split || s.nseg == 0 || cap > ((int64_t)16 << 20) || !s.repeatable) {
         s.part_cap = 0;
         return;
     }

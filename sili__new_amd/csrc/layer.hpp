@@ -160,6 +160,9 @@ struct DScatter {
     // entries' places in this store (built for a layer that trains)
     std::vector<ColBlocks<DScatter>> cblk;
     DevBuf<uint32_t> from;
+    // SILI_SPLIT_COMBINE=1 when it was built: its user wants the same bits from
+    // every call, so no kernel takes over that orders the sums otherwise
+    bool repeatable = false;
     // split rows combined in item order by the float4 gather: arrivals per
     // row (rows+1, zero between launches) and per-item partial sums
     // (part_cap floats; empty: combined by atomics)

@@ -974,7 +974,7 @@ bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int sk
     const auto gain = [&] { return 0.9 * other - mfma24_us(Shape(s), B); };
     if (mode != 2) {
         // few rows: not a block for every CU
-        if (s.rows < 2048 || ((B == 2 || B == 4 || B == 8) && env_int("SILI_B1_STREAM", 1) == 2)) return false;
+        if (s.repeatable || s.rows < 2048 || ((B == 2 || B == 4 || B == 8) && env_int("SILI_B1_STREAM", 1) == 2)) return false;
         const double g = gain();
         if (Shape(s).cells * 0.375 > 8e9 || g < 0) return false;
         s.m24_saved += g + 0.1 * other;

@@ -204,6 +204,19 @@ def test_mfma24_is_built_when_it_pays(hip, monkeypatch):
     assert all("fwd:mfma24" not in kernel_counts(hip, small, lambda: small.forward_dense(xs)) for _ in range(20))
 
 
+def test_mfma24_leaves_repeatable_stores_alone(hip, monkeypatch):
+    """A store built for bitwise repeats gives the same bits on every call."""
+    monkeypatch.delenv("SILI_MFMA24", raising=False)
+    monkeypatch.setenv("SILI_SPLIT_COMBINE", "1")
+    L = make(hip, 1000, 8192, 0.3, 6, False, full=False)[1]
+    rng = np.random.default_rng(7)
+    x = rng.normal(size=(128, 1000)).astype(np.float32)
+    y = L.forward_dense(x)
+    for _ in range(60):
+        assert np.array_equal(L.forward_dense(x).view(np.uint32), y.view(np.uint32))
+    assert "fwd:mfma24" not in kernel_counts(hip, L, lambda: L.forward_dense(x))
+
+
 def test_mfma24_leaves_what_a_captured_call_needs(hip, monkeypatch):
     """A batch that ran twice before it is captured: the captured call takes the
     other kernels, whose first use builds and waits, so the first of those runs
