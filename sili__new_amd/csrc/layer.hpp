@@ -133,7 +133,7 @@ struct DScatter {
     DevBuf<uint8_t> slc_col;
     DevBuf<uint32_t> slc_off;
     int64_t slc_w = 0, slc_n = 0;
-    // the 2:4 copy of the matrix-core gather (mfma24.hip; built on first use,
+    // the 2:4 copy of the matrix-core gather (mfma24.hip; built once it pays,
     // dropped when values or structure change): FP4 codes and positions per 32
     // rows x 128 columns, and the entries that a group of 4 columns has no
     // place for, by row
@@ -146,12 +146,20 @@ struct DScatter {
     // us it saved or would have saved since the values last changed, and when
     // to build it: m24_saved >= m24_cost * m24_wait
     double m24_saved = 0, m24_cost = 0, m24_wait = 1;
+    void free_m24() {
+        m24_val.reset();
+        m24_idx.reset();
+        m24_ovf.reset();
+    }
     // batches that the other kernels have served since then: what they build on
     // first use is there, so a call under stream capture, which takes them,
     // builds nothing
     std::bitset<513> m24_warm;
+    // (one that was dropped before it had paid gives its memory back: the next
+    // may be a long time off)
     void drop_m24() {
         if (m24_valid) m24_wait = m24_saved < m24_cost * (m24_wait + 1) ? std::min(m24_wait * 2, 1e6) : 1;
+        if (m24_wait > 1) free_m24();
         m24_valid = false;
         m24_saved = 0;
         m24_warm.reset();

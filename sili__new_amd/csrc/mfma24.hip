@@ -894,14 +894,13 @@ double others_us(const DScatter &s, int64_t B) {
 
 // The other gathers serve this layer until its structure changes.
 static void release(DScatter &s) {
-    s.m24_val.reset();
-    s.m24_idx.reset();
-    s.m24_ovf.reset();
+    s.free_m24();
     s.m24_valid = false;
     s.m24_failed = true;
 }
 
-// The copy and the workspace of batch B; false: no memory for them.
+// The copy and the workspace of batch B; false: no memory for them (the copy
+// takes SILI_MFMA24_FREE_PCT percent of the free memory at most).
 static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
     const int64_t ntile = (s.rows + 31) / 32, nkb = n_blocks(s.cols);
     const size_t ops = (size_t)(nkb * 4 * operand_tiles(B) * (B <= SMALL_B ? 1 : 3) * 1024);
@@ -914,6 +913,15 @@ static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
             L.m24_epoch = 0;
         }
         if (s.m24_valid) return true;
+        // a copy takes a part of what is free at most, so that those of many
+        // layers leave room for everything else on the device
+        size_t free = 0, all = 0;
+        SILI_HIP(hipMemGetInfo(&free, &all));
+        const double bytes = (double)(ntile * nkb) * 64.0 * 24.0 + 9.0 * (double)s.nnz;  // with what its building takes
+        if (bytes > 0.01 * env_int("SILI_MFMA24_FREE_PCT", 25) * (double)free) {
+            release(s);
+            return false;
+        }
         ProfScope ps("mfma24_build", st);
         s.m24_val.ensure((size_t)(ntile * nkb * 64));
         s.m24_idx.ensure((size_t)(ntile * nkb * 64));

@@ -204,6 +204,39 @@ def test_mfma24_is_built_when_it_pays(hip, monkeypatch):
     assert all("fwd:mfma24" not in kernel_counts(hip, small, lambda: small.forward_dense(xs)) for _ in range(20))
 
 
+def test_mfma24_copy_gives_its_memory_back(hip, monkeypatch):
+    """A copy of 50 MB and more that an update drops before it has paid is freed;
+    one that is too large a part of the free memory is not built."""
+    lib = C.CDLL(hip.LIB_PATH)
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    monkeypatch.delenv("SILI_MFMA24", raising=False)
+    L = make(hip, 2048, 65536, 0.1, 9, False, full=False)[1]
+    rng = np.random.default_rng(9)
+    x, dy = rng.normal(size=(128, 2048)).astype(np.float32), rng.normal(size=(128, 65536)).astype(np.float32)
+    L.forward_dense(x)
+    L.backward_dense(dy, 0.01)  # the optimizer's state
+    for _ in range(30):
+        if kernel_counts(hip, L, lambda: L.forward_dense(x)).get("fwd:mfma24"):
+            break
+    else:
+        pytest.fail("no copy was built")
+    held = free()
+    for _ in range(10):  # (the runtime gives freed memory back some calls later)
+        L.backward_dense(dy, 0.01)
+        kernel_counts(hip, L, lambda: L.forward_dense(x))
+        if free() - held > 45 << 20:
+            break
+    assert free() - held > 45 << 20
+    monkeypatch.setenv("SILI_MFMA24_FREE_PCT", "0")
+    for _ in range(60):
+        assert "fwd:mfma24" not in kernel_counts(hip, L, lambda: L.forward_dense(x))
+
+
 def test_mfma24_leaves_repeatable_stores_alone(hip, monkeypatch):
     """A store built for bitwise repeats gives the same bits on every call."""
     monkeypatch.delenv("SILI_MFMA24", raising=False)
