@@ -392,7 +392,24 @@ struct Scratch {
 // NoScalePolicy (SparseLinearLayerNoScale).
 enum UpdateVariant : int { UPDATE_PLAIN = 0, UPDATE_RESYNC = 1, UPDATE_NOSCALE = 2 };
 
+// Work issued on one stream from here on comes after what another one has now.
+struct StreamOrder {
+    hipEvent_t ev = nullptr;
+    StreamOrder() = default;
+    StreamOrder(const StreamOrder &) = delete;
+    StreamOrder &operator=(const StreamOrder &) = delete;
+    ~StreamOrder() {
+        if (ev) (void)hipEventDestroy(ev);
+    }
+    void after(hipStream_t later, hipStream_t earlier) {
+        if (!ev) SILI_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        SILI_HIP(hipEventRecord(ev, earlier));
+        SILI_HIP(hipStreamWaitEvent(later, ev, 0));
+    }
+};
+
 struct Layer {
+    StreamOrder order;
     int device = 0;
     hipStream_t stream = nullptr;
     int64_t n_in = 0, n_out = 0, max_weights = 0;
@@ -710,9 +727,11 @@ inline bool capturing(hipStream_t st) {
 }
 
 // Before a copy of the store's values is built on the layer's stream for a call
-// on st: an update that st still runs has to have written them.
-inline void finish_updates(const Layer &L, hipStream_t st) {
-    if (st != L.stream) SILI_HIP(hipStreamSynchronize(st));
+// on st: an update that st still runs writes them first, and a gather that it
+// still runs has read the copy that is there.  (The layer's stream waits, not
+// the host, which goes on issuing the build.)
+inline void finish_updates(Layer &L, hipStream_t st) {
+    if (st != L.stream) L.order.after(L.stream, st);
 }
 
 // The copies of s in K blocks of width (block) columns, holding the store's

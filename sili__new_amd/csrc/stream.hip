@@ -735,9 +735,9 @@ StreamShape stream_shape(int nb, int64_t nwin, int64_t nx, int xmode) {
 }
 
 // Build d = the stream copy of s cut into K column blocks of cb columns
-// (device work on L's stream; synchronous).  Sets d.failed when a block
-// would not keep 31-bit offsets.
-void build_stream(Layer &L, const DScatter &s, DStream &d, int K, int64_t cb) {
+// for a call on stream call_st (device work on L's stream; synchronous).  Sets
+// d.failed when a block would not keep 31-bit offsets.
+void build_stream(Layer &L, const DScatter &s, DStream &d, int K, int64_t cb, hipStream_t call_st) {
     hipStream_t st = L.stream;
     const int64_t rows = s.rows;
     d.valid = false;
@@ -796,6 +796,8 @@ void build_stream(Layer &L, const DScatter &s, DStream &d, int K, int64_t cb) {
     d.ne_row.ensure(ne_off + 1);
     d.ne_start.ensure(ne_off + 1);
     d.win.ensure(win_off + 1);
+    // (the places above depend on no value: they run beside a queued update)
+    finish_updates(L, call_st);
     SILI_HIP(hipMemsetAsync(d.idx.p, 0, off + WIN_BYTES, st));
     SILI_HIP(hipMemsetAsync(d.val.p, 0, off + WIN_BYTES, st));
     for (int k = 0; k < K; ++k) {
@@ -877,16 +879,12 @@ void stream_gather(Layer &L, DScatter &s, const ScaleView &sc, const float *in, 
     DStream *d = nullptr;
     if (K == 1) {
         d = &s.stream1;
-        if (!d->valid && !d->failed) {
-            finish_updates(L, st);
-            build_stream(L, s, *d, 1, s.cols);
-        }
+        if (!d->valid && !d->failed) build_stream(L, s, *d, 1, s.cols, st);
     } else {
         d = &s.streamK;
         if (!d->valid || d->K != K || d->cb != cb) {
             d->failed = false;
-            finish_updates(L, st);
-            build_stream(L, s, *d, K, cb);
+            build_stream(L, s, *d, K, cb, st);
         }
     }
     if (!d->valid) throw_error(3, "stream copy exceeds 2 GiB");
