@@ -973,11 +973,12 @@ static bool ensure_mfma24(Layer &L, DScatter &s, int64_t B, hipStream_t st) {
 // The first call of each batch takes the other kernels, which leaves a program
 // that runs a batch before it captures it all that the captured call needs.
 bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int skip, hipStream_t st) {
+    if (B < 2 || B > MAX_B || s.cols > (int64_t(1) << 21)) return false;
+    if (s.nnz == 0 || s.m24_failed || L.has_nonfinite || skip != SKIP_NONE || sc.rank != 1) return false;
     // SILI_MFMA24 (read per call): 0 never, 2 whenever it can and at once, 1
     // (default) by the estimates
     const int mode = env_int("SILI_MFMA24", 1);
-    if (mode == 0 || s.nnz == 0 || s.m24_failed || L.has_nonfinite || skip != SKIP_NONE || sc.rank != 1) return false;
-    if (B < 2 || B > MAX_B || s.cols > (int64_t(1) << 21)) return false;
+    if (mode == 0) return false;
     const double other = others_us(s, B);
     const auto gain = [&] { return 0.9 * other - mfma24_us(Shape(s), B); };
     if (mode != 2) {
