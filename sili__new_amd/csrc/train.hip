@@ -233,8 +233,10 @@ __device__ __forceinline__ void reduce8(const float *sred, float *rdx, int64_t b
 // step as written, the others (the caller's `mode`, uniform over the wave) are
 // fast ones: save() and back() keep and restore the lane's state around a
 // group of them, and redo() says, for the whole wave, that the group must be
-// run as written.  sx: 16-byte aligned.
-template <typename Step, typename Save, typename Back, typename Redo>
+// run as written.  sx: 16-byte aligned.  FEW: batches up to FEW_STEPS, which have
+// none of the groups.
+constexpr int64_t FEW_STEPS = 3;
+template <bool FEW, typename Step, typename Save, typename Back, typename Redo>
 __device__ __forceinline__ void batch_steps(const float *__restrict__ gcol, int64_t B, const float *sx, float *rdx,
                                             float *sred, int mode, Step &step, Save &save, Back &back, Redo &redo) {
     const uint32_t lane = __lane_id();
@@ -268,19 +270,21 @@ __device__ __forceinline__ void batch_steps(const float *__restrict__ gcol, int6
         }
         reduce8(sred, rdx, b0, N);
     };
-    const float4 z4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float4 n0 = B >= 4 ? load_f4(gcol) : z4;
-    float4 n1 = B >= 8 ? load_f4(gcol + 4) : z4;
     int64_t b0 = 0;
-    for (; b0 + 8 <= B; b0 += 8) {
-        const float4 c0 = n0, c1 = n1;
-        if (b0 + 12 <= B) n0 = load_f4(gcol + b0 + 8);
-        if (b0 + 16 <= B) n1 = load_f4(gcol + b0 + 12);
-        group(std::integral_constant<int, 8>{}, b0, c0, c1);
-    }
-    if (b0 + 4 <= B) {
-        group(std::integral_constant<int, 4>{}, b0, n0, z4);
-        b0 += 4;
+    if constexpr (!FEW) {
+        const float4 z4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float4 n0 = B >= 4 ? load_f4(gcol) : z4;
+        float4 n1 = B >= 8 ? load_f4(gcol + 4) : z4;
+        for (; b0 + 8 <= B; b0 += 8) {
+            const float4 c0 = n0, c1 = n1;
+            if (b0 + 12 <= B) n0 = load_f4(gcol + b0 + 8);
+            if (b0 + 16 <= B) n1 = load_f4(gcol + b0 + 12);
+            group(std::integral_constant<int, 8>{}, b0, c0, c1);
+        }
+        if (b0 + 4 <= B) {
+            group(std::integral_constant<int, 4>{}, b0, n0, z4);
+            b0 += 4;
+        }
     }
     for (; b0 < B; ++b0) {
         const float tot = wave_sum(step(std::integral_constant<int, 0>{}, b0, sx[b0], gcol[b0]));
@@ -323,7 +327,7 @@ struct TrainArgs {
 //   DeferredScaleWrite: the true-units weight cw = code * vs0 * os0 is
 //     stepped by g; scale gradients weigh by the stored code, component 0
 //     only; (cw, ci) are kept for k_train_store (linear_disldo.hpp:687-790).
-template <int RANK, bool DEFERRED, bool COLS>
+template <int RANK, bool DEFERRED, bool COLS, bool FEW>
 __global__ __launch_bounds__(256, RANK == 1 ? 4 : 2) void k_train_rows(TrainArgs a) {
     __shared__ double s_part[WAVES_T][64][2 * RANK];
     extern __shared__ __attribute__((aligned(16))) float s_dyn[];  // [wave][dx B | x B]
@@ -458,8 +462,8 @@ __global__ __launch_bounds__(256, RANK == 1 ? 4 : 2) void k_train_rows(TrainArgs
             }
         };
         auto redo = [&]() -> bool { return __any(has && rg.outside()); };
-        const int mode = a.fast && __all(ok) ? (os1 ? 2 : 1) : 0;
-        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, mode, step, save, back, redo);
+        const int mode = !FEW && a.fast && __all(ok) ? (os1 ? 2 : 1) : 0;
+        batch_steps<FEW>(a.gT + (int64_t)col * B, B, sx, rdx, sred, mode, step, save, back, redo);
         if (has) {
             if (deferred) {
                 a.def_w[vb] = wv;
@@ -630,7 +634,7 @@ __global__ __launch_bounds__(256) void k_sparse_train_rows(SparseTrainArgs a) {
         };
         auto nothing = []() {};
         auto never = []() -> bool { return false; };
-        batch_steps(a.gT + (int64_t)col * B, B, sx, rdx, sred, 1, step, nothing, nothing, never);
+        batch_steps<false>(a.gT + (int64_t)col * B, B, sx, rdx, sred, 1, step, nothing, nothing, never);
         if (has) a.val[vb] = (uint8_t)byte;
         s_part[wave][lane][0] = has ? psg : 0.0;
         s_part[wave][lane][1] = has ? psgc : 0.0;
@@ -717,6 +721,39 @@ struct B4TrainArgs {
 // the 4 rows' reads of one step group fall into different banks.
 constexpr uint32_t TURN_LD = 20;  // a (row, step)'s 16 tiles in LDS, 16-byte aligned
 __host__ __device__ inline int64_t b4_ld(int64_t B) { return ((B + 3) & ~(int64_t)3) + 4; }
+
+// The scale step of a canonical row that block4 tiles cover, component k
+// (linear_disldo.hpp:1923-1951), from the sums over its tiles.
+__device__ __forceinline__ void b4_scale_step(const B4TrainArgs &a, int64_t i, double sum, double sum_c, float vs,
+                                              float imp, uint32_t step, float pow_step, float scale_eff_lr) {
+    if (sum == 0.0 && sum_c == 0.0) return;
+    const float g_agg = (float)sum, contrib_agg = (float)sum_c;
+    if (!finite_f(g_agg) || !finite_f(contrib_agg)) return;
+    const float new_vs_imp = a.beta2 * imp + (1.0f - a.beta2) * (g_agg * g_agg + contrib_agg * contrib_agg);
+    if (!finite_f(new_vs_imp)) return;
+    a.vs_step[i] = step;
+    const float bias_correction = 1.0f - pow_step;
+    const float hat = bias_correction > 0.0f ? new_vs_imp / bias_correction : new_vs_imp;
+    if (!finite_f(hat)) return;
+    const float new_vs = vs - scale_eff_lr * g_agg / (__builtin_sqrtf(hat) + a.eps);
+    if (!finite_f(new_vs)) return;
+    a.vs_imp[i] = new_vs_imp;
+    a.vs[i] = new_vs;
+}
+// A trained slot's byte: importance and code, each rounded to nearest or by its
+// own draw.
+__device__ __forceinline__ uint8_t b4_slot_byte(const B4TrainArgs &a, uint64_t t, uint32_t slot, float q, float imp) {
+    uint32_t wq, iq;
+    if (a.stochastic) {
+        const uint64_t base = a.seed + 2ull * ((uint64_t)a.nnz_scattered + t * 16 + slot);
+        wq = fp4_encode_stochastic(q, splitmix64(base));
+        iq = fp4_encode_stochastic(imp, splitmix64(base + 1ull));
+    } else {
+        wq = fp4_encode(q);
+        iq = fp4_encode(imp);
+    }
+    return (uint8_t)((iq << 4) | wq);
+}
 
 // A lane's state while its 4 slots train.
 template <int RANK, bool COLS>
@@ -945,16 +982,7 @@ __global__ __launch_bounds__(64 * W, RANK == 1 && !COLS ? 4 : 2) void k_train_b4
                 if (!has[j]) continue;
                 const uint32_t slot = (uint32_t)j * 4u + li;
                 const float imp = s.ci[j] / (imp_scale * (a.ois ? a.ois[c0 + j] : 1.0f));
-                uint32_t wq, iq;
-                if (a.stochastic) {
-                    const uint64_t base = a.seed + 2ull * ((uint64_t)a.nnz_scattered + (uint64_t)t * 16 + slot);
-                    wq = fp4_encode_stochastic(s.q[j], splitmix64(base));
-                    iq = fp4_encode_stochastic(imp, splitmix64(base + 1ull));
-                } else {
-                    wq = fp4_encode(s.q[j]);
-                    iq = fp4_encode(imp);
-                }
-                a.tiles[(uint64_t)t * 16 + slot] = (uint8_t)((iq << 4) | wq);
+                a.tiles[(uint64_t)t * 16 + slot] = b4_slot_byte(a, t, slot, s.q[j], imp);
                 if constexpr (COLS) {
 #pragma unroll
                     for (int k = 0; k < 2 * RANK; ++k) a.b4term[((uint64_t)t * 16 + slot) * 2 * RANK + k] = s.mc[j][k];
@@ -988,24 +1016,151 @@ __global__ __launch_bounds__(64 * W, RANK == 1 && !COLS ? 4 : 2) void k_train_b4
         const float scale_eff_lr = a.lr / (float)nnz_row;
 #pragma unroll
         for (int k = 0; k < RANK; ++k) {
-            const double sum = s_row[threadIdx.x][k], sum_c = s_row[threadIdx.x][RANK + k];
-            if (sum == 0.0 && sum_c == 0.0) continue;
-            const float g_agg = (float)sum, contrib_agg = (float)sum_c;
-            if (!finite_f(g_agg) || !finite_f(contrib_agg)) continue;
             const int64_t i = r * RANK + k;
-            const float new_vs_imp = a.beta2 * a.vs_imp[i] + (1.0f - a.beta2) * (g_agg * g_agg + contrib_agg * contrib_agg);
-            if (!finite_f(new_vs_imp)) continue;
             const uint32_t step = a.vs_step[i] + 1u;
-            a.vs_step[i] = step;
-            const float bias_correction = 1.0f - a.pow_tab[step];
-            const float hat = bias_correction > 0.0f ? new_vs_imp / bias_correction : new_vs_imp;
-            if (!finite_f(hat)) continue;
-            const float new_vs = a.vs[i] - scale_eff_lr * g_agg / (__builtin_sqrtf(hat) + a.eps);
-            if (!finite_f(new_vs)) continue;
-            a.vs_imp[i] = new_vs_imp;
-            a.vs[i] = new_vs;
+            b4_scale_step(a, i, s_row[threadIdx.x][k], s_row[threadIdx.x][RANK + k], a.vs[i], a.vs_imp[i], step,
+                          a.pow_tab[step], scale_eff_lr);
         }
     }
+}
+
+// Lane J of the calling lane's quad (DPP quad_perm, a VALU move), and ((l0 + l1)
+// + l2) + l3 over the quad, on every lane of it.
+template <int J>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), J * 0x55, 0xF, 0xF, false));
+}
+template <int J>
+__device__ __forceinline__ double quad_lane(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, J * 0x55, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), J * 0x55, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ float quad_sum(float v) {
+    return ((quad_lane<0>(v) + quad_lane<1>(v)) + quad_lane<2>(v)) + quad_lane<3>(v);
+}
+
+// k_train_b4 for batches of 1 to 3, whose few steps fill no lane's time: a slot a
+// lane (lane = 16 * tile + 4 * li + lj, a quad is a tile row), 16 tiles a block
+// at a time, the steps as written.  What bounds it is the chain from the tile's
+// column to its gradient to its row's scale step, so what the row's step and dx
+// start from is loaded beside the rest.  The same sums in the same order.
+// Training step, us, k_train_b4 / this one at batch 1, 2, 3: 9216 x 2816 with 8.5
+// tiles a row 46.9 / 38.3, 47.0 / 44.0, 48.5 / 44.0; 6144 x 4096 with 20 51.9 /
+// 43.8 at batch 2; 16384 x 16384 with 123 156 / 130 at batch 2.
+template <int RANK, bool COLS>
+__global__ __launch_bounds__(256) void k_train_b4_few(B4TrainArgs a) {
+    constexpr uint32_t TILES = 16;
+    __shared__ double s_mr[TILES][4][2 * RANK];
+    __shared__ float s_turn[FEW_STEPS][TILES][4];  // the tile rows' dx terms
+    const uint32_t lane = threadIdx.x & 63u, tl = threadIdx.x >> 4, li = (lane >> 2) & 3u, lj = lane & 3u;
+    const int64_t br = blockIdx.x;
+    const uint32_t t0 = a.tile_start[br], t1 = a.tile_start[br + 1];
+    if (t0 == t1) return;  // the whole block
+    const int B = (int)a.B;
+    const int64_t row = br * 4 + li;
+    const bool row_ok = row < a.n_in;
+    // thread (l, k) sums row l's scale terms k, thread 64 + (step, l) its dx, in tile order
+    const uint32_t ml = threadIdx.x / (2u * RANK), mk = threadIdx.x % (2u * RANK);
+    const uint32_t ds = (threadIdx.x - 64u) >> 2, dl = threadIdx.x & 3u;
+    const bool sums_m = threadIdx.x < 8u * RANK && br * 4 + ml < a.n_in;
+    const bool sums_dx = threadIdx.x - 64u < 4u * (uint32_t)B && br * 4 + dl < a.n_in;
+    float *const dx = a.dx + (sums_dx ? (int64_t)ds * a.n_in + br * 4 + dl : 0);
+    const float dx_0 = sums_dx ? *dx : 0.0f;
+    const int64_t si = (br * 4 + ml) * RANK + mk;  // (mk < RANK: the thread that steps the scale)
+    const bool steps = sums_m && mk < (uint32_t)RANK;
+    const float vs_0 = steps ? a.vs[si] : 0.0f, imp_0 = steps ? a.vs_imp[si] : 0.0f;
+    const uint32_t step_0 = steps ? a.vs_step[si] + 1u : 0u;
+    const float pow_0 = a.pow_tab[step_0];
+    float vs_k[RANK], x[FEW_STEPS];
+#pragma unroll
+    for (int k = 0; k < RANK; ++k) vs_k[k] = row_ok ? a.vs[row * RANK + k] : 0.0f;
+    const float imp_scale = (a.is && row_ok) ? a.is[row] : 1.0f;
+#pragma unroll
+    for (int b = 0; b < FEW_STEPS; ++b) x[b] = b < B && row_ok ? a.xT[row * B + b] : 0.0f;
+    const uint32_t nnz_row = (t1 - t0) * 4u;
+    const float eff_lr = a.lr_per_row_nnz ? a.lr / (float)nnz_row : a.lr;
+    double msum = 0.0;
+    float dsum = 0.0f;
+    for (uint32_t p0 = t0; p0 < t1; p0 += TILES) {
+        const bool tile_ok = p0 + tl < t1;
+        const uint32_t t = tile_ok ? p0 + tl : p0;
+        const int64_t c0 = (int64_t)a.tcol[t] * 4, col = c0 + lj;
+        const bool full = c0 + 4 <= a.n_out, has = tile_ok && row_ok && col < a.n_out;
+        const uint32_t slot = lj * 4u + li;
+        const uint32_t byte = has ? (uint32_t)a.tiles[(uint64_t)t * 16 + slot] : 0u;
+        float dy[FEW_STEPS], os_k[RANK], S = 0.0f;
+#pragma unroll
+        for (int b = 0; b < FEW_STEPS; ++b) dy[b] = b < B && has ? a.gT[col * B + b] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < RANK; ++k) {
+            os_k[k] = has ? a.os[col * RANK + k] : 0.0f;
+            S = S + vs_k[k] * os_k[k];
+        }
+        const float cis = imp_scale * ((a.ois && has) ? a.ois[col] : 1.0f);
+        const float q0 = fp4_decode(byte & 0xFu);
+        float q = q0, ci = fp4_decode(byte >> 4) * cis;
+        double mr[2 * RANK];
+        float mc[2 * RANK];
+#pragma unroll
+        for (int k = 0; k < 2 * RANK; ++k) {
+            mr[k] = 0.0;
+            mc[k] = 0.0f;
+        }
+#pragma unroll
+        for (int b = 0; b < FEW_STEPS; ++b) {
+            if (b >= B) break;
+            const float iv = x[b], dyv = dy[b], g = dyv * iv, contrib = q0 * iv;
+            ci = bounded_update_ci(ci, g, contrib, a.beta2, a.min_decay_frac, a.max_ci);
+            q = q + bounded_update_cw(g, ci, S, eff_lr, a.eps, a.damp != 0, a.max_abs_delta);
+            const float qf = (q == 0.0f) ? a.zero_escape_eps : q;
+            const float d = quad_sum(has ? (q * S) * dyv : 0.0f);
+            if (lj == 0u) s_turn[b][tl][li] = d;
+#pragma unroll
+            for (int k = 0; k < RANK; ++k) {
+                if constexpr (COLS) {
+                    mc[k] = mc[k] + (qf * vs_k[k]) * g;
+                    mc[RANK + k] = mc[RANK + k] + (qf * vs_k[k]) * contrib;
+                }
+                if (full) {  // (uniform over a quad)
+                    mr[k] = mr[k] + (double)quad_sum((qf * os_k[k]) * g);
+                    mr[RANK + k] = mr[RANK + k] + (double)quad_sum((qf * os_k[k]) * contrib);
+                } else {
+                    const double d0 = has ? ((double)qf * (double)os_k[k]) * (double)g : 0.0;
+                    const double d1 = has ? ((double)qf * (double)os_k[k]) * (double)contrib : 0.0;
+                    mr[k] = (((mr[k] + quad_lane<0>(d0)) + quad_lane<1>(d0)) + quad_lane<2>(d0)) + quad_lane<3>(d0);
+                    mr[RANK + k] = (((mr[RANK + k] + quad_lane<0>(d1)) + quad_lane<1>(d1)) + quad_lane<2>(d1)) + quad_lane<3>(d1);
+                }
+            }
+        }
+        if (lj == 0u) {
+#pragma unroll
+            for (int k = 0; k < 2 * RANK; ++k) s_mr[tl][li][k] = mr[k];
+        }
+        __syncthreads();
+        const uint32_t n = min(TILES, t1 - p0);
+        if (sums_m) {
+#pragma unroll 4
+            for (uint32_t u = 0; u < n; ++u) msum = msum + s_mr[u][ml][mk];
+        }
+        if (sums_dx) {
+#pragma unroll 4
+            for (uint32_t u = 0; u < n; ++u) dsum = dsum + s_turn[ds][u][dl];
+        }
+        if (has) {
+            a.tiles[(uint64_t)t * 16 + slot] = b4_slot_byte(a, t, slot, q, ci / cis);
+            if constexpr (COLS) {
+#pragma unroll
+                for (int k = 0; k < 2 * RANK; ++k) a.b4term[((uint64_t)t * 16 + slot) * 2 * RANK + k] = mc[k];
+            }
+        }
+        __syncthreads();
+    }
+    if (sums_dx) *dx = dx_0 + dsum;
+    // the row's two sums are in neighbouring blocks of RANK lanes
+    const double msum_c = __shfl_down(msum, RANK, 64);
+    if (steps) b4_scale_step(a, si, msum, msum_c, vs_0, imp_0, step_0, pow_0, a.lr / (float)nnz_row);
 }
 
 // ---- the block rows' write-back with eviction --------------------------------
@@ -1444,13 +1599,20 @@ inline unsigned nblk(int64_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 template <int RANK>
 void launch_rows_rank(bool deferred, bool cols, dim3 grid, dim3 block, uint32_t lds, hipStream_t st,
                       const TrainArgs &a) {
-    if (deferred) {
-        if (cols) launch(k_train_rows<RANK, true, true>, grid, block, lds, st, a);
-        else launch(k_train_rows<RANK, true, false>, grid, block, lds, st, a);
-    } else {
-        if (cols) launch(k_train_rows<RANK, false, true>, grid, block, lds, st, a);
-        else launch(k_train_rows<RANK, false, false>, grid, block, lds, st, a);
-    }
+    // (the kernel with the fast groups, which batches of 1 to 3 have none of,
+    // took 11.6 us there, the one without 11.3: 2816 x 2048, batch 1)
+    auto go = [&](auto few) {
+        constexpr bool F = decltype(few)::value;
+        if (deferred) {
+            if (cols) launch(k_train_rows<RANK, true, true, F>, grid, block, lds, st, a);
+            else launch(k_train_rows<RANK, true, false, F>, grid, block, lds, st, a);
+        } else {
+            if (cols) launch(k_train_rows<RANK, false, true, F>, grid, block, lds, st, a);
+            else launch(k_train_rows<RANK, false, false, F>, grid, block, lds, st, a);
+        }
+    };
+    if (a.B <= FEW_STEPS) go(std::true_type{});
+    else go(std::false_type{});
 }
 
 void launch_rows_kernel(int rank, bool deferred, bool cols, dim3 grid, dim3 block, uint32_t lds, hipStream_t st,
@@ -1465,9 +1627,14 @@ void launch_rows_kernel(int rank, bool deferred, bool cols, dim3 grid, dim3 bloc
 
 // One wave a block while a row has at most a wave's 16 tiles on average, else 4.
 // Training step, 9216 x 2816 with 8.5 tiles a row, us: with 4 waves / with 1:
-// batch 1 57.7 / 46.9, 2 57.9 / 47.0, 5 63.6 / 51.9, 13 77.0 / 63.8.
+// batch 5 63.6 / 51.9, 13 77.0 / 63.8.  Batches up to FEW_STEPS take k_train_b4_few.
 template <int RANK>
 void launch_b4_rank(const B4TrainArgs &a, int64_t ntiles, hipStream_t st) {
+    if (a.B <= FEW_STEPS) {
+        if (a.b4term) launch((k_train_b4_few<RANK, true>), dim3((unsigned)a.brows), dim3(256), 0, st, a);
+        else launch((k_train_b4_few<RANK, false>), dim3((unsigned)a.brows), dim3(256), 0, st, a);
+        return;
+    }
     const uint32_t waves = ntiles <= 16 * a.brows ? 1u : 4u;
     // x and each wave's dx rows: up to 82 KB at batch 1024
     const uint32_t lds = (uint32_t)((1 + waves) * 4 * b4_ld(a.B) * sizeof(float));

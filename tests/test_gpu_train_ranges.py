@@ -78,3 +78,14 @@ def test_block4_update_ranges(hip, kind, shape):
         b4_reserve_like_device(L, H, 64 + 16 * len(c["br"]))
         x, dy = batch_inputs(c["rng"], B, n_in, n_out, kind)
         check(L, H, x, dy, 0.05, kind, True, f"{kind} {shape} batch {B}")
+
+
+@pytest.mark.parametrize("B", [1, 2, 3])
+@pytest.mark.parametrize("rank", [1, 2, 3, 4])
+def test_block4_few_steps(hip, monkeypatch, rank, B):
+    """Batches of 1 to 3 (a slot a lane): every rank, output scales that train,
+    rows past a block's 16 tiles, an edge tile and an edge row."""
+    import test_gpu_train as T
+    opts = dict(rank=rank, os_trainable=True, imp_scales=True, tile_density=0.7)
+    monkeypatch.setattr(T, "B4_CASES", [(39, 150, 0.01, 70 + 3 * rank + B, B, 0.3, opts, "plain")])
+    T.test_block4_update_matches_oracle(hip, 0)
