@@ -729,9 +729,10 @@ inline bool capturing(hipStream_t st) {
 // Before a copy of the store's values is built on the layer's stream for a call
 // on st: an update that st still runs writes them first, and a gather that it
 // still runs has read the copy that is there.  (The layer's stream waits, not
-// the host, which goes on issuing the build.)
+// the host, which goes on issuing the build.  A wait for a stream under a
+// relaxed capture would draw the build into the graph.)
 inline void finish_updates(Layer &L, hipStream_t st) {
-    if (st != L.stream) L.order.after(L.stream, st);
+    if (st != L.stream && !capturing(st)) L.order.after(L.stream, st);
 }
 
 // The copies of s in K blocks of width (block) columns, holding the store's

@@ -33,9 +33,9 @@ class Calls:
     def forward(self, B):
         self.rt("sili_forward_dense", self.h, self.x, B, self.y, self.st)
 
-    def capture(self, B):
+    def capture(self, B, mode=0):
         g, run = C.c_void_p(), C.c_void_p()
-        self.rt("hipStreamBeginCapture", self.st, 0)
+        self.rt("hipStreamBeginCapture", self.st, mode)
         self.forward(B)
         self.rt("hipStreamEndCapture", self.st, C.byref(g))
         self.rt("hipGraphInstantiate", C.byref(run), g, None, None, C.c_size_t(0))
@@ -156,6 +156,24 @@ def test_capture_of_a_batch_that_never_ran(hip, cold):
     close_to(calls.result(replay, x), want, "replay")
     close_to(calls.result(lambda: calls.forward(cold), x), want, "eager")
     close_to(calls.result(replay, x), want, "replay")
+    calls.close()
+
+
+def test_relaxed_capture_builds_a_stream_copy(hip, monkeypatch):
+    """A relaxed capture (mode 2) may allocate and wait on other streams: the
+    stream copy of batch 8 is built beside it, on the layer's stream."""
+    L, plain = twins(hip)
+    rng = np.random.default_rng(9)
+    calls = Calls(hip, L, N_IN, N_OUT, B)
+    calls.result(lambda: calls.forward(B), rng.normal(size=(B, N_IN)).astype(np.float32))
+    x = rng.normal(size=(8, N_IN)).astype(np.float32)
+    want = plain.forward_dense(x)
+    monkeypatch.setenv("SILI_B1_STREAM", "2")
+    replay = calls.capture(8, 2)
+    assert L.info()["stream_shadow"] == 1
+    for _ in range(3):
+        close_to(calls.result(replay, x), want, "replay")
+        close_to(calls.result(lambda: calls.forward(8), x), want, "eager")
     calls.close()
 
 
