@@ -1013,13 +1013,12 @@ def run_layer_config(a, hip, api, rt, cfg, steps, warmup, train_lr, synapto_reps
                 "traffic": None if train_lr else measured_traffic(dom_name, cfg), "avg_op_ms": round(dom_avg_ms, 5),
                 "launches_per_op": launches, "algorithmic_bytes": dom_bytes}
         if dom_name == "bwd:train_rows":
-            # one synapse's batch steps are a dependent chain of ~80 VALU
-            # instructions each (correctly rounded sqrt and division, clamps,
-            # fp64 gradient terms): the kernel is bound by instruction issue
-            steps = nnz_s * B
-            roof["synapse_steps_per_s"] = round(steps / (dom_avg_ms * 1e-3), 1)
-            roof["note"] = ("k_train_rows is bound by VALU issue (~80 instructions per synapse per batch step, "
-                            "4 cycles per 64-lane instruction per SIMD), not by HBM")
+            # one synapse's batch steps are a dependent chain of VALU
+            # instructions (correctly rounded sqrt and division, clamps, fp64
+            # gradient terms): the kernel is bound by instruction issue
+            roof["synapse_steps_per_s"] = round(nnz_s * B / (dom_avg_ms * 1e-3), 1)
+            roof["note"] = ("k_train_rows is bound by VALU issue (55 instructions per wave and batch step, counted "
+                            "over the whole kernel, 4 cycles each per SIMD), not by HBM")
         if cfg == 0:
             step_bytes = alg["fwd:gather"]
             flops = 2 * units * B
