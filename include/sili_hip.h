@@ -382,7 +382,7 @@ typedef struct {
     int32_t pad0;
     int64_t short_rows_canonical; /* short rows (whole rows of <= 28 index bytes) the float4
                                      gather packs up to 16 to a wave, canonical store (0 until
-                                     a gather at batch 4..64 has used them, or when fewer than a
+                                     a gather at batch 2..64 has used them, or when fewer than a
                                      quarter of the work items are such rows) */
     int64_t short_rows_shadow;    /* ... of the shadow store */
 } sili_info;

@@ -220,8 +220,8 @@ constexpr int64_t BATCH_SLACK = 4;
 
 // out[b*out_ld + row] for b < nb: scattered gather (stores; atomics for split
 // rows -- then the caller has zeroed out).  in is feature-major in[c*in_ld + b].
-// accumulate: add to out (batches with nb % 4 == 0 and aligned feature-major
-// input only; used by the column-block passes).
+// accumulate: add to out (batches above 1 and inputs below 2 GiB only; used by
+// the column-block passes).
 void launch_gather(const GatherPlan &p, const ScaleView &sc, const float *in, int64_t in_ld,
                    float *out, int64_t out_ld, int64_t nb, int skip, hipStream_t st, bool accumulate = false);
 // Block4 contribution, added into out.

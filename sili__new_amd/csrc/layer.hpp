@@ -755,8 +755,9 @@ bool staged_wanted(const DScatter &s, int64_t B);
 void launch_gather_staged(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t B, float *out,
                           int64_t out_ld, hipStream_t st);
 // The matrix-core gather (mfma24.hip): whether it takes this case (its copy of
-// the store is then built), and out[b, r] for every row r of s (written).  in: batch-major [B][in_ld], inT: the same feature-major, which
-// the call itself fills when xT == inT is given (NULL: filled before).
+// the store is then built), and out[b, r] for every row r of s (written).  in:
+// batch-major [B][in_ld], inT: the same feature-major, which the call itself
+// fills when xT == inT is given (NULL: filled before).
 bool mfma24_wanted(Layer &L, DScatter &s, const ScaleView &sc, int64_t B, int skip, hipStream_t st);
 void launch_mfma24(Layer &L, DScatter &s, const ScaleView &sc, const float *in, int64_t in_ld, const float *inT,
                    float *xT, int64_t B, float *out, int64_t out_ld, hipStream_t st);

@@ -553,10 +553,10 @@ __device__ __forceinline__ void add_overflow(const M24Args &a, float *col, uint3
 // stages of 24 KiB, two stages ahead in a ring of three, so that two blocks (4
 // waves per SIMD) share a CU (MT = 4 with one block a CU was behind at every
 // size).  Each wave reads an operand once per MT products; MT = 1 is for
-// layers of few blocks.  What
-// bounds it now is the issue of the products and their LDS reads: 424 us for
-// 0.8 PFLOP of stored-form products, 1.9 of the 4.16 PFLOP/s the instruction
-// reaches alone.  A operands come straight from the copy, a 128-column block
+// layers of few blocks.  What it waits for (5120 x 204800, 10 %, batch 128, 481
+// us): no unit is busy throughout -- the matrix cores 39 % of the cycles, the
+// CU's load path (operand stages and the copy) 66, LDS 22, VALU issue 17, HBM at
+// 1.6 TB/s; a block's waves meet at a barrier per stage.  A operands come straight from the copy, a 128-column block
 // ahead, and are issued behind the stage loads of their block, so that waiting
 // for a stage does not wait for them.
 template <int MT, int WN>
@@ -671,7 +671,9 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
 
 // Batches up to 21: the 3 pieces are operand columns of their own (3 B <= 32
 // NT), so one product per row tile and 32 columns serves the whole batch, and
-// the copy's bytes are what is waited for: 4 waves of MT row tiles each share
+// the copy's bytes are what is waited for (4.3 TB/s at 5120 x 204800, batch 8, 5.5
+// at 1310720 rows; the load path busy 58 % of the cycles, the matrix cores 13): 4
+// waves of MT row tiles each share
 // the B operands (a 128-column block per stage, in a ring of four), and read
 // their A operands three blocks ahead.
 constexpr int SMALL_B = 21;
@@ -845,7 +847,7 @@ namespace {
 // to 16384^2, 5120 x 16384, 4096 x 65536, 1024 x 100000 and 5120 x 204800 at
 // densities 0.01 to 0.1 and batches 4 to 128; the dispatch below compares them
 // and takes the matrix cores where they are ahead by a tenth.  Both sides as
-// measured (other path / this one):
+// measured, us (other path / this one):
 //   5120 x 204800, 10 %: batch 4 62 / 97, 8 128 / 99, 16 552 / 135, 32 678 / 153,
 //     64 1196 / 248, 128 1339 / 464
 //   16384^2, 2 %: 16 39 / 67, 32 44 / 98, 64 77 / 114, 128 167 (segments) / 163;

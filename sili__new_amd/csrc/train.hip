@@ -121,18 +121,19 @@ __device__ __forceinline__ uint32_t requantize(float w, float imp, bool stochast
 }
 
 // ---- the step without IEEE fix-ups ------------------------------------------
-// A synapse's batch step is bound by VALU issue: of the ~90 instructions that
-// the expressions above compile to, 27 are the IEEE square root and division
+// A synapse's batch step is bound by VALU issue: of the instructions that the
+// expressions above compile to, 27 are the IEEE square root and division
 // with their scaling, rounding and special-case selects.  The fast step keeps
 // only what an operand in the middle of the exponent range needs -- the
 // sequences below give the same correctly rounded results there -- and
 // records what the operands' ranges were; a group of steps that met anything
 // else (a tiny, negative, infinite or NaN second moment, a tiny step
 // numerator) is run again from its saved state with the expressions as
-// written.  8192 x 8192, 1.34 M synapses, batch 64: k_train_rows 232 -> 184 us
-// (40 VALU instructions per synapse-step, two of them transcendental);
+// written.  8192 x 8192, 1.34 M synapses, batch 64: k_train_rows 213 -> 170 us,
+// 78 -> 55 VALU instructions a wave and batch step (SQ_INSTS_VALU over the whole
+// kernel; 79 % of the issue slots, and two of the 55 are transcendental);
 // 16384 x 16384, 504 K tiles, batch 256, with the lane layout described at
-// k_train_b4: 6.33 -> 2.80 ms.
+// k_train_b4: 6.33 -> 2.74 ms, 98 -> 50 instructions per 64 slots and step (95 %).
 
 // sqrt of x == 0 or x in [2^-80, 2^80]: v_rsq_f32 (1 ulp) and Markstein's
 // correction by the exact remainder x - s*s.  Equal to the IEEE root for every
@@ -705,8 +706,8 @@ struct B4TrainArgs {
 // 4 slots are 4 independent chains of batch steps, and the sums over a tile
 // row that the reference's 4-lane path forms, ((t0 + t1) + t2) + t3 in fp32
 // per batch step for the row gradient, stay inside the lane.  (A slot per lane
-// with the sums by quad moves spent 21 of its 87 instructions per slot-step on
-// them, and each batch step added its dx terms to LDS by itself.)  An edge
+// with the sums by quad moves spent 21 instructions per slot-step on them, and
+// each batch step added its dx terms to LDS by itself.)  An edge
 // tile, whose 4 columns are not all in range, adds its fp64 row-gradient terms
 // one by one (the reference's scalar path).  The tiles' fp64 row partials are
 // added in tile order; then the block rows' scale step.  dx: per 4 batch steps

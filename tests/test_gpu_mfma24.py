@@ -3,8 +3,10 @@ the oracle (linear_disldo.hpp:68-126 and its transpose) where they can go
 wrong: rows and columns that fill no tile of 32 or block of 128 (512 columns a
 turn), empty rows, groups of 4 columns with 3 and 4 entries (the overflow list)
 up to full rows, batches around the operand tiles (10 and 21 for the pieces as
-columns, 32, 64, 128 a chunk), inputs without an exact split (non-finite, tiny),
-and the copy's life: built late, dropped when values or structure change."""
+columns, 32, 64, 128 a chunk), inputs over the whole float range (tiny ones that
+take the products, large and non-finite ones that leave them, scales that cancel),
+and the copy's life: built late, dropped when values or structure change, its
+memory, stores and captured calls that stay with the other kernels."""
 import ctypes as C
 
 import numpy as np
