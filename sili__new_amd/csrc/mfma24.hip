@@ -556,9 +556,9 @@ __device__ __forceinline__ void add_overflow(const M24Args &a, float *col, uint3
 // layers of few blocks.  What it waits for (5120 x 204800, 10 %, batch 128, 481
 // us): no unit is busy throughout -- the matrix cores 39 % of the cycles, the
 // CU's load path (operand stages and the copy) 66, LDS 22, VALU issue 17, HBM at
-// 1.6 TB/s; a block's waves meet at a barrier per stage.  A operands come straight from the copy, a 128-column block
-// ahead, and are issued behind the stage loads of their block, so that waiting
-// for a stage does not wait for them.
+// 1.6 TB/s; a block's waves meet at a barrier per stage.  A operands come
+// straight from the copy, a 128-column block ahead, and are issued behind the
+// stage loads of their block, so that waiting for a stage does not wait for them.
 template <int MT, int WN>
 __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
     constexpr int WM = 8 / WN, SPS = 4 / WN;                   // row groups; steps per stage
@@ -673,9 +673,8 @@ __global__ __launch_bounds__(512, 4) void k_m24(M24Args a) {
 // NT), so one product per row tile and 32 columns serves the whole batch, and
 // the copy's bytes are what is waited for (4.3 TB/s at 5120 x 204800, batch 8, 5.5
 // at 1310720 rows; the load path busy 58 % of the cycles, the matrix cores 13): 4
-// waves of MT row tiles each share
-// the B operands (a 128-column block per stage, in a ring of four), and read
-// their A operands three blocks ahead.
+// waves of MT row tiles each share the B operands (a 128-column block per stage,
+// in a ring of four), and read their A operands three blocks ahead.
 constexpr int SMALL_B = 21;
 // 32 rows of a wave, all batch rows: the pieces' sums, then the overflow
 // entries of a row by the two lanes that hold it (half h: batch rows [h
